@@ -1,0 +1,122 @@
+"""The reciprocal Ewald sum on the matrix cores (csrc/ewald_recip.hip) where
+its tiles end: ions around the 32 of an LDS chunk and the 64 of a workgroup,
+k ranges around the 4 x 4 columns and the 8 and 4 wide tiles of n3, more n3
+than one item holds (96), sheared cells (off-centre ranges of n3), and no k at
+all; against the oracle, and against sums in 80-bit arithmetic.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from atomistica_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+RC, BETA = 4.0, 0.55
+REL = 1e-10
+
+
+def _cell(shape, shear=0.0):
+    return np.diag(np.asarray(shape, float)) @ np.array([[1.0, 0, 0], [shear, 1.0, 0], [-0.6 * shear, 0.8 * shear, 1.0]])
+
+
+def _ions(n, cell, seed):
+    rng = np.random.default_rng(seed)
+    # some ions outside the cell: phases are taken modulo whole turns
+    pos = (rng.random((n, 3)) + rng.integers(-2, 3, (n, 3))) @ cell
+    q = rng.normal(size=n)
+    return pos, q - q.mean()
+
+
+def _oracle(pos, cell, q, kmax):
+    nl = O.nl_build(pos, cell, [True] * 3, RC, avgn=2000)
+    a, b = O.ewald_real(pos, q, cell, nl, RC, BETA), O.ewald_kspace(pos, q, cell, BETA, kmax)
+    return [x + y for x, y in zip(a, b)]
+
+
+def _close(a, b):
+    a, b = np.asarray(a), np.asarray(b)
+    return np.abs(a - b).max() <= REL * max(1.0, np.abs(b).max())
+
+
+CASES = [
+    (1, (6.0, 6.5, 7.0), 0.0, 3.0), (2, (6.0, 6.0, 6.0), 0.0, 1.06), (2, (5.0, 5.0, 5.0), 0.0, 0.5),
+    (31, (9.0, 8.0, 7.0), 0.3, 3.0), (32, (9.0, 8.0, 7.0), 0.0, 3.1), (33, (11.0, 8.0, 13.0), -0.4, 2.9),
+    (63, (12.0, 12.0, 12.0), 0.0, 2.5), (64, (12.0, 13.0, 12.0), 0.2, 4.2), (65, (12.0, 12.0, 15.0), 0.0, 3.3),
+    (129, (20.0, 9.0, 9.0), 0.1, 3.0),
+    # n3 up to 111: two items per patch, the second one short; and up to 192
+    (40, (7.0, 7.0, 230.0), 0.0, 3.05), (17, (6.0, 6.0, 400.0), 0.0, 3.03),
+    # long first and second axes
+    (20, (180.0, 6.0, 6.0), 0.0, 3.0), (20, (6.0, 180.0, 6.0), 0.05, 3.0),
+]
+
+
+@pytest.mark.parametrize("n,shape,shear,kmax", CASES)
+def test_recip_edges(n, shape, shear, kmax):
+    from atomistica_amd import native as N
+    cell = _cell(shape, shear)
+    pos, q = _ions(n, cell, 11 * n)
+    print("ewald recip: %d ions, cell %s shear %g kmax %g" % (n, shape, shear, kmax), flush=True)
+    p = N.from_atoms(pos, cell, [True] * 3, np.full(n, 11, np.int32))
+    nl = N.Neighbors(2000)
+    pot = N.Ewald(cutoff=RC, beta=BETA, kmax=kmax)
+    pot.bind_to(p, nl)
+    e, f, w = pot.energy_and_forces(p, nl, q)
+    phi = pot.potential(p, nl, q)
+    re_, rf, rw, rp = _oracle(pos, cell, q, kmax)
+    assert abs(e - re_) <= REL * max(1.0, abs(re_))
+    assert _close(f, rf) and _close(w, rw) and _close(phi, rp)
+
+
+def test_recip_edges_batched():
+    from atomistica_amd.batch import Batch, ewald_batch
+    kmax = 3.05
+    S, qs = [], []
+    for n, shape, shear, _ in CASES:
+        cell = _cell(shape, shear)
+        pos, q = _ions(n, cell, 13 * n)
+        S.append((pos, cell))
+        qs.append(q)
+    b = Batch(S)
+    e, f, w, phi = (t.cpu().numpy() for t in ewald_batch(b, np.concatenate(qs), RC, BETA, kmax, phi=True))
+    for s, (pos, cell) in enumerate(S):
+        re_, rf, rw, rp = _oracle(pos, cell, qs[s], kmax)
+        a = slice(b.offsets[s], b.offsets[s + 1])
+        assert abs(e[s] - re_) <= REL * max(1.0, abs(re_)), s
+        assert _close(f[a], rf) and _close(w[s], rw) and _close(phi[a], rp), s
+
+
+def test_recip_forces_against_80_bit_sums():
+    """512 ions, n up to 12: a phase 2 pi n s carries n 2 pi 2^-54 of s's
+    rounding, 4e-15 at n = 12, and a force sums some hundred large terms of
+    either sign; twelve times that is allowed."""
+    from atomistica_amd import native as N
+    LD = np.longdouble
+    pos, cell, pbc, Z, q = W.rocksalt(4, sigma=0.1, seed=9)
+    beta = W.ewald_beta(10.0, 1e-8)
+    kmax = W.ewald_kmax(beta, 1e-8)
+    nl = N.Neighbors(220)
+    p = N.from_atoms(pos, cell, pbc, Z)
+    pot = N.Ewald(cutoff=10.0, beta=beta, kmax=kmax)
+    pot.bind_to(p, nl)
+    _, f, _ = pot.energy_and_forces(p, nl, q)
+    ref = O.ewald_real(pos, q, cell, O.nl_build(pos, cell, pbc, 10.0, avgn=400), 10.0, beta)[1].astype(LD)
+    L = cell[0, 0].astype(LD)
+    nmax = int(kmax * float(L) / (2 * np.pi)) + 1
+    n = np.stack(np.meshgrid(*[np.arange(-nmax, nmax + 1)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    half = (n[:, 0] > 0) | ((n[:, 0] == 0) & ((n[:, 1] > 0) | ((n[:, 1] == 0) & (n[:, 2] > 0))))
+    n = n[half & ((2 * np.pi / float(L)) ** 2 * (n ** 2).sum(1) <= kmax * kmax)]
+    pi = LD("3.14159265358979323846264338327950288")
+    for c in range(0, len(n), 512):
+        m = n[c:c + 512]
+        t = m.astype(LD) @ (pos.astype(LD) / L).T
+        ph = 2 * pi * (t - np.rint(t))
+        co, si = np.cos(ph), np.sin(ph)
+        a, b = co @ q.astype(LD), si @ q.astype(LD)
+        k2 = (2 * pi / L) ** 2 * (m ** 2).sum(1)
+        w = np.exp(-k2 / (4 * LD(beta) ** 2)) / k2
+        im = (w * a)[:, None] * si - (w * b)[:, None] * co
+        ref += 8 * pi / L ** 3 * q.astype(LD)[:, None] * (2 * pi / L) * (im.T @ m.astype(LD))
+    err = float(np.sqrt(((f - ref) ** 2).sum() / (ref ** 2).sum()))
+    print("ewald forces, 512 ions: relative error against 80-bit sums %.2e" % err, flush=True)
+    assert err < 5e-14
