@@ -296,7 +296,7 @@ __device__ __forceinline__ void row_stats_wave(int longest, int last, int2 *__re
     if ((threadIdx.x & 63) == 0) part[w] = make_int2(longest, last);
 }
 
-// One wavefront per block of B x B x B home bins (B = 1 for dense bins).
+// nsub wavefronts per block of B x B x B home bins (B = 1 for dense bins).
 // The block's candidates -- the atoms of its (B + 2 nd)^3 stencil bins in
 // x-major bin order, ascending atom order inside each bin -- are held in
 // registers, 256 per pass (lane L holds candidates L, L+64, L+128, L+192).
@@ -308,10 +308,11 @@ __device__ __forceinline__ void row_stats_wave(int longest, int last, int2 *__re
 // accepted pair inside the row; rows go to a padded staging area (stride S
 // per sorted slot, neighbours by slot).
 // MULTI: blocks of B > 1 bins, whose candidates are checked against each home
-// atom's own stencil
+// atom's own stencil.  nsub wavefronts share a block's home atoms; a row is
+// one wavefront's, so the share does not change it.
 template <bool ORTHO, bool MULTI>
 __global__ void __launch_bounds__(256)
-k_bin_pairs(int B, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__restrict__ atoms,
+k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__restrict__ atoms,
             const int *__restrict__ cell_start, int *__restrict__ scnt,
             int2 *__restrict__ stage, int S, int *__restrict__ flags, int2 *__restrict__ part)
 {
@@ -319,10 +320,12 @@ k_bin_pairs(int B, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__r
     NlShared &L = sh[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
     const int nbx = (g.nc[0] + B - 1) / B, nby = (g.nc[1] + B - 1) / B, nbz = (g.nc[2] + B - 1) / B;
-    const int blk = xcd_block() * NL_WAVES + (threadIdx.x >> 6);
+    // wavefront sub of nsub takes its share of the block's home atoms
+    const int wid = xcd_block() * NL_WAVES + (threadIdx.x >> 6);
+    const int blk = wid / nsub, sub = wid - blk * nsub;
     // every wavefront of the grid leaves its row-statistics record
     if (blk >= nbx * nby * nbz) {
-        if (lane == 0) part[blk] = make_int2(0, 0);
+        if (lane == 0) part[wid] = make_int2(0, 0);
         return;
     }
     const int bz = blk % nbz, by = (blk / nbz) % nby, bx = blk / (nbz * nby);
@@ -347,9 +350,10 @@ k_bin_pairs(int B, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__r
         int v = __shfl_up(hpre, o, 64);
         if (lane >= o) hpre += v;
     }
-    const int MH = __shfl(hpre, 63, 64);
-    if (MH == 0) {
-        if (lane == 0) part[blk] = make_int2(0, 0);
+    const int MHB = __shfl(hpre, 63, 64);
+    const int M0 = (int)((long long)MHB * sub / nsub), MH = (int)((long long)MHB * (sub + 1) / nsub);
+    if (MH <= M0) {
+        if (lane == 0) part[wid] = make_int2(0, 0);
         return;
     }
     const int sx = B + 2 * g.nd[0], sy = B + 2 * g.nd[1], sz = B + 2 * g.nd[2];
@@ -357,7 +361,7 @@ k_bin_pairs(int B, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__r
     int wmax = 0, wlast = 0;
     bool stage_over = false, img_bad = false;
 
-    for (int a0 = 0; a0 < MH; a0 += NL_HMAX) {
+    for (int a0 = M0; a0 < MH; a0 += NL_HMAX) {
         const int ma = min(NL_HMAX, MH - a0);
         __builtin_amdgcn_wave_barrier();
         L.pre[lane] = hpre;
@@ -551,7 +555,7 @@ k_bin_pairs(int B, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__r
             if (c > S) stage_over = true;
         }
     }
-    row_stats_wave(wmax, wlast, part, blk);
+    row_stats_wave(wmax, wlast, part, wid);
     const bool any_over = __ballot(stage_over) != 0ull;
     const bool any_bad = __ballot(img_bad) != 0ull;
     if (lane == 0 && any_over) atomicOr(flags, DERR_STAGE_OVERFLOW);
@@ -1161,7 +1165,18 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
         const bool ortho = C.A[1] == 0.0 && C.A[2] == 0.0 && C.A[3] == 0.0 && C.A[5] == 0.0 &&
                            C.A[6] == 0.0 && C.A[7] == 0.0;
         const long long nblk_b = (long long)((g.nc[0] + B - 1) / B) * ((g.nc[1] + B - 1) / B) * ((g.nc[2] + B - 1) / B);
-        const int nbin_blk = (int)((nblk_b + NL_WAVES - 1) / NL_WAVES);
+        // Wavefronts per block of bins.  A wavefront loads the block's
+        // candidates and walks its share of the home atoms, so sharing costs
+        // a candidate load per wavefront and pays while the chip is not full:
+        // up to 2048 wavefronts whatever their share (1200 ions at r_c = 10,
+        // 27 blocks of 44 atoms: 451 -> 55 us; 6048 Cu atoms, 315 of 19:
+        // 56 -> 24 us), up to 8192 while each keeps 16 home atoms (216 000
+        // ions, 4096 of 53: 451 -> 407 us with 2, 466 with 6).  64 000 atoms
+        // in 4913 blocks of 13: 57 us with 1, 67 with 2.
+        const double homes = per_bin * B * B * B;
+        const int nsub = (int)std::max(1.0, std::max(std::min(2048.0 / (double)nblk_b, homes),
+                                                     std::min(8192.0 / (double)nblk_b, homes / 16.0)));
+        const int nbin_blk = (int)((nblk_b * nsub + NL_WAVES - 1) / NL_WAVES);
         // staging stride: expected neighbours from the density, grown on demand
         if (nl->stage_w <= 0) {
             const double *A = p->cell.A;
@@ -1190,7 +1205,7 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
         } else {
             auto kern = ortho ? (B > 1 ? k_bin_pairs<true, true> : k_bin_pairs<true, false>)
                               : (B > 1 ? k_bin_pairs<false, true> : k_bin_pairs<false, false>);
-            AGPU_LAUNCH("nl_pairs", kern, dim3(nbin_blk), dim3(TB), 0, s, B, g, C, cutoff_sq,
+            AGPU_LAUNCH("nl_pairs", kern, dim3(nbin_blk), dim3(TB), 0, s, B, nsub, g, C, cutoff_sq,
                         nl->atoms_sorted.as<SortedAtom>(), nl->cell_start.as<int>(), nl->scnt.as<int>(),
                         nl->stage.as<int2>(), S, flags + 3, part);
         }

@@ -287,3 +287,25 @@ def test_tersoff_deferred_list_check_redo():
         assert _close(f, ref[1]) and _close(w, ref[2])
         if per_at:
             assert _close(epa, ref[3]) and _close(wpa, ref[4])
+
+
+def _equal_oracle(pos, cell, pbc, rc, avgn):
+    p = N.from_atoms(pos, cell, pbc, np.full(len(pos), 14, np.int32))
+    nl = N.Neighbors(avgn)
+    nl.request_interaction_range(rc)
+    off, j, dc = nl.get_list(p)
+    ro, rj, rdc = O.nl_build(pos, cell, pbc, rc, avgn=avgn)
+    assert np.array_equal(off, ro) and np.array_equal(j, rj) and np.array_equal(dc, rdc)
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 63, 64, 65, 130, 700])
+@pytest.mark.parametrize("shear", [0.0, 0.25])
+def test_shared_home_atoms_of_a_bin_block(n, shear):
+    """Dense bins of few atoms in all: each block's home atoms are shared by
+    as many wavefronts as it has atoms, or as the chip still takes."""
+    rng = np.random.default_rng(n)
+    cell = np.diag([11.0, 13.0, 17.5]) @ np.array([[1, 0, 0], [shear, 1, 0], [0, -shear, 1.0]])
+    pos = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))) @ cell
+    print("shared home atoms", n, shear, flush=True)
+    _equal_oracle(pos, cell, [True] * 3, 5.5, 800)
+    _equal_oracle(pos, cell, [True, False, True], 5.5, 800)
