@@ -21,8 +21,9 @@
 //                  neighbours named by slot, and the row counts by slot.
 //                  k_bin_pairs (a wavefront per block of home bins,
 //                  candidates shared by the wavefront) when bins are dense,
-//                  k_atom_pairs (a thread per home atom) when they hold < 4
-//                  atoms.  The force kernels read these rows and the slot
+//                  k_atom_pairs (a thread per home atom; k_column_pairs,
+//                  nine lanes per home atom, for fewer atoms) when they hold
+//                  < 4 atoms.  The force kernels read these rows and the slot
 //                  records directly (bin-order storage: a neighbour's
 //                  position is a slot record near the home atom's own).
 //   5. exclusive scan of the counts -> slot row offsets; the caller-order
@@ -778,6 +779,203 @@ k_atom_pairs(int nat, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *
     }
 }
 
+// The same search with nine lanes per home atom, one per z column of a
+// 3 x 3 x 3 stencil (7 atoms per wavefront): lane k walks column
+// k = 3 (ox + 1) + (oy + 1), its accepted candidates are counted and marked,
+// the counts of the lanes before it in stencil order give its place in the
+// row, and a second walk over the marked candidates writes them.  The lanes'
+// walks take turns where the thread-per-atom kernel walks nine columns one
+// after the other.
+constexpr int NL_COLS = 9;
+constexpr int NL_CPW = 7;       // home atoms per wavefront
+
+template <bool ORTHO>
+__global__ void __launch_bounds__(256)
+k_column_pairs(int nat, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__restrict__ atoms,
+               const float4 *__restrict__ pos32, const int *__restrict__ cell_start, int *__restrict__ scnt,
+               int2 *__restrict__ stage, int S, int *__restrict__ flags, int2 *__restrict__ part)
+{
+    const int lane = threadIdx.x & 63, a = lane / NL_COLS, k = lane - a * NL_COLS;
+    const int p = (xcd_block() * 4 + (threadIdx.x >> 6)) * NL_CPW + a;
+    bool bad = false;
+    int cnt = 0, ih = 0;
+    unsigned long long mark = 0;
+    float hx0 = 0.f, hy0 = 0.f, hz0 = 0.f, hm = 0.f;
+    int w0 = 0, w1 = 0, w2 = 0, ux = 0, uy = 0;
+    int q0[3] = {0, 0, 0}, q1[3] = {0, 0, 0};
+    const float rc = (float)sqrt(cutoff_sq);
+    const bool act = a < NL_CPW && p < nat;
+    if (act) {
+        const float4 H = pos32[p];
+        const SortedAtom A = atoms[p];
+        const double ri[3] = {A.x, A.y, A.z};
+        int hc[3], hw[3];
+        bin_of(g, ri, hc, hw);
+        dc_unpack(A.w, w0, w1, w2);
+        ih = A.j;
+        hx0 = H.x;
+        hy0 = H.y;
+        hz0 = H.z;
+        hm = fabsf(H.w);
+        const int nz = g.nc[2], zlo = hc[2] - 1, zhi = hc[2] + 1;
+        int cx = hc[0] + k / 3 - 1, cy = hc[1] + k % 3 - 1;
+        bool ok = true;
+        if (g.pbc[0]) {
+            if (cx < 1) { cx += g.nc[0]; ux = 1; }
+            else if (cx > g.nc[0]) { cx -= g.nc[0]; ux = -1; }
+        } else {
+            ok = cx >= 1 && cx <= g.nc[0];
+        }
+        if (g.pbc[1]) {
+            if (cy < 1) { cy += g.nc[1]; uy = 1; }
+            else if (cy > g.nc[1]) { cy -= g.nc[1]; uy = -1; }
+        } else {
+            ok = ok && cy >= 1 && cy <= g.nc[1];
+        }
+        if (ok) {
+            // wrapped from the top (u_z = +1), unwrapped, wrapped from the bottom (u_z = -1)
+            const int bc = ((cx - 1) * g.nc[1] + (cy - 1)) * nz;
+            q0[1] = cell_start[bc + max(zlo, 1) - 1];
+            q1[1] = cell_start[bc + min(zhi, nz)];
+            if (g.pbc[2] && zlo < 1) {
+                q0[0] = cell_start[bc + zlo + nz - 1];
+                q1[0] = cell_start[bc + nz];
+            }
+            if (g.pbc[2] && zhi > nz) {
+                q0[2] = cell_start[bc];
+                q1[2] = cell_start[bc + zhi - nz];
+            }
+        }
+    }
+    // one candidate: the image code of an accepted one, -1 beyond the packed
+    // range, -2 when it is no neighbour
+    auto test = [&](int q, const float4 B, int uz, float hx, float hy, float hz, float e0) -> int {
+        const float dx = hx - B.x, dy = hy - B.y, dz = hz - B.z;
+        const float d2f = dx * dx + dy * dy + dz * dz;
+        const float E2 = 2.0f * (e0 + 4.76837158e-7f * fmaxf(hm, fabsf(B.w)));
+        const float th = rc + E2, tl = rc - E2;
+        const bool exact = !(E2 < 2e-3f * rc);
+        if (!exact && !(d2f < th * th * 1.000001f)) return -2;
+        int s0 = w0 + ux, s1 = w1 + uy, s2 = w2 + uz;
+        if (__float_as_int(B.w) < 0) {
+            int v0, v1, v2;
+            dc_unpack(atoms[q].w, v0, v1, v2);
+            s0 -= v0;
+            s1 -= v1;
+            s2 -= v2;
+        }
+        if (q == p && s0 == 0 && s1 == 0 && s2 == 0) return -2;
+        if (exact || !(d2f < tl * tl * 0.999999f)) {
+            const SortedAtom Ap = atoms[p], Bq = atoms[q];
+            if (!(pair_d2<ORTHO>(C, Ap.x, Ap.y, Ap.z, Bq.x, Bq.y, Bq.z, s0, s1, s2) < cutoff_sq)) return -2;
+        }
+        if (!dc_pack_ok(s0) || !dc_pack_ok(s1) || !dc_pack_ok(s2)) return -1;
+        return dc_pack(s0, s1, s2);
+    };
+    int seen = 0;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        if (q0[t] >= q1[t]) continue;
+        double au[3];
+        if (ORTHO) {
+            au[0] = C.A[0] * (double)ux;
+            au[1] = C.A[4] * (double)uy;
+            au[2] = C.A[8] * (double)(1 - t);
+        } else {
+            for (int x = 0; x < 3; ++x) au[x] = image_x(C, x, ux, uy, 1 - t);
+        }
+        const float hx = hx0 + (float)au[0], hy = hy0 + (float)au[1], hz = hz0 + (float)au[2];
+        const float e0 = 5.9604645e-8f * (4.0f * (float)(fabs(au[0]) + fabs(au[1]) + fabs(au[2])) + 8.0f * rc);
+        for (int q = q0[t]; q < q1[t]; q += 2) {
+            const float4 B0 = pos32[q], B1 = pos32[min(q + 1, q1[t] - 1)];
+            const int c0 = test(q, B0, 1 - t, hx, hy, hz, e0);
+            const int c1 = q + 1 < q1[t] ? test(q + 1, B1, 1 - t, hx, hy, hz, e0) : -2;
+            if (c0 > -2) {
+                ++cnt;
+                bad = bad || c0 < 0;
+                if (seen < 64) mark |= 1ull << seen;
+            }
+            if (c1 > -2) {
+                ++cnt;
+                bad = bad || c1 < 0;
+                if (seen + 1 < 64) mark |= 1ull << (seen + 1);
+            }
+            seen += min(2, q1[t] - q);
+        }
+    }
+    // this lane's place in the row: the counts of the columns before it
+    int at = 0, total = 0;
+#pragma unroll
+    for (int c = 0; c < NL_COLS; ++c) {
+        const int v = __shfl(cnt, a * NL_COLS + c, 64);
+        at += c < k ? v : 0;
+        total += v;
+    }
+    if (act) {
+        int2 *row = stage + (size_t)p * S;
+        seen = 0;
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const int n = max(q1[t] - q0[t], 0);
+            if (cnt > 0 && n > 0) {
+                if (seen + n <= 64) {
+                    // the marked ones only
+                    unsigned long long m = (mark >> seen) & (n < 64 ? (1ull << n) - 1 : ~0ull);
+                    while (m) {
+                        const int q = q0[t] + __ffsll((long long)m) - 1;
+                        m &= m - 1;
+                        int s0 = w0 + ux, s1 = w1 + uy, s2 = w2 + 1 - t;
+                        if (__float_as_int(pos32[q].w) < 0) {
+                            int v0, v1, v2;
+                            dc_unpack(atoms[q].w, v0, v1, v2);
+                            s0 -= v0;
+                            s1 -= v1;
+                            s2 -= v2;
+                        }
+                        if (at < S) row[at] = make_int2(q, dc_pack(s0, s1, s2));
+                        ++at;
+                    }
+                } else {
+                    // a column of more than 64 candidates: tested again
+                    double au[3];
+                    for (int x = 0; x < 3; ++x) au[x] = image_x(C, x, ux, uy, 1 - t);
+                    const float hx = hx0 + (float)au[0], hy = hy0 + (float)au[1], hz = hz0 + (float)au[2];
+                    const float e0 =
+                        5.9604645e-8f * (4.0f * (float)(fabs(au[0]) + fabs(au[1]) + fabs(au[2])) + 8.0f * rc);
+                    for (int q = q0[t]; q < q1[t]; ++q) {
+                        const int c = test(q, pos32[q], 1 - t, hx, hy, hz, e0);
+                        if (c <= -2) continue;
+                        if (at < S) row[at] = make_int2(q, c);
+                        ++at;
+                    }
+                }
+            }
+            seen += n;
+        }
+        if (k == 0) scnt[p] = total;
+    }
+    // one row-statistics record per block
+    {
+        __shared__ int2 sm[4];
+        int longest = act ? total : 0, last = act && total > 0 ? ih + 1 : 0;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) {
+            longest = max(longest, __shfl_xor(longest, o, 64));
+            last = max(last, __shfl_xor(last, o, 64));
+        }
+        if (lane == 0) sm[threadIdx.x >> 6] = make_int2(longest, last);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            part[blockIdx.x] = make_int2(max(max(sm[0].x, sm[1].x), max(sm[2].x, sm[3].x)),
+                                         max(max(sm[0].y, sm[1].y), max(sm[2].y, sm[3].y)));
+    }
+    const unsigned long long mo = __ballot(act && total > S), mb = __ballot(bad);
+    if (lane == 0) {
+        if (mo) atomicOr(flags, DERR_STAGE_OVERFLOW);
+        if (mb) atomicOr(flags, DERR_IMAGE_RANGE);
+    }
+}
+
 // Copy staged rows (sorted slot p, stride S, neighbours by slot) into the
 // CSR rows of the caller atoms, neighbours by caller index (nothing when the
 // build overflowed).
@@ -1190,10 +1388,21 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
         // row-statistics records: one per block (thread per atom) or per
         // wavefront (wavefront per bin block)
         const int na = (nat + TB - 1) / TB;
-        const int npart = per_atom ? na : nbin_blk * NL_WAVES;
+        // Nine lanes per atom while a thread per atom leaves the chip idle:
+        // 512 Si atoms 47 -> 13 us, 39 000 (triclinic) 42 -> 20, 64 000
+        // 42 -> 24, 100 000 C/H 40 -> 30, but 216 000 48 -> 55 and 1 000 000
+        // 150 -> 209 (a lane's column is over before its group's longest).
+        const bool columns =
+            per_atom && nat < 150000 && g.nd[0] == 1 && g.nd[1] == 1 && g.nd[2] == 1 && (!g.pbc[2] || g.nc[2] >= 3);
+        const int nc = (nat + 4 * NL_CPW - 1) / (4 * NL_CPW);
+        const int npart = columns ? nc : per_atom ? na : nbin_blk * NL_WAVES;
         AGPU_CHECK(nl->part.reserve(sizeof(int2) * (size_t)npart));
         int2 *part = nl->part.as<int2>();
-        if (per_atom) {
+        if (columns) {
+            AGPU_LAUNCH("nl_pairs", (ortho ? k_column_pairs<true> : k_column_pairs<false>), dim3(nc), dim3(TB), 0, s,
+                        nat, g, C, cutoff_sq, nl->atoms_sorted.as<SortedAtom>(), nl->pos32.as<float4>(),
+                        nl->cell_start.as<int>(), nl->scnt.as<int>(), nl->stage.as<int2>(), S, flags + 3, part);
+        } else if (per_atom) {
             if (ortho)
                 AGPU_LAUNCH("nl_pairs", k_atom_pairs<true>, dim3(na), dim3(TB), 0, s, nat, g, C, cutoff_sq,
                             nl->atoms_sorted.as<SortedAtom>(), nl->pos32.as<float4>(), nl->cell_start.as<int>(),

@@ -309,3 +309,20 @@ def test_shared_home_atoms_of_a_bin_block(n, shear):
     print("shared home atoms", n, shear, flush=True)
     _equal_oracle(pos, cell, [True] * 3, 5.5, 800)
     _equal_oracle(pos, cell, [True, False, True], 5.5, 800)
+
+
+@pytest.mark.parametrize("n", [1, 6, 7, 8, 27, 28, 29, 300])
+@pytest.mark.parametrize("shear", [0.0, 0.2])
+@pytest.mark.parametrize("pbc", [[True] * 3, [True, True, False], [False, False, True]])
+def test_column_search(n, shear, pbc):
+    """Sparse bins of few atoms: nine lanes per home atom, 7 atoms per
+    wavefront and 28 per workgroup; one cluster of 120 atoms in a bin fills
+    columns beyond the 64 candidates that a lane marks."""
+    rng = np.random.default_rng(3 * n)
+    cell = np.diag([17.0, 22.0, 31.0]) @ np.array([[1, 0, 0], [shear, 1, 0], [0, -shear, 1.0]])
+    pos = rng.random((n, 3)) @ cell
+    print("column search", n, shear, pbc, flush=True)
+    _equal_oracle(pos, cell, pbc, 3.0, 400)
+    if n == 300:
+        q = np.concatenate([pos, (np.array([0.02, 0.5, 0.97]) + 0.02 * rng.random((120, 3))) @ cell])
+        _equal_oracle(q, cell, pbc, 3.0, 400)
