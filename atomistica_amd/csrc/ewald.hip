@@ -4,7 +4,7 @@
 // (src/potentials/coulomb/pme.f90:215-321, 386-437, 467-472): erfc(beta r)/r
 // over every neighbour image inside the cutoff, charges with |q| <= 1e-10
 // skipped, self energy -beta/sqrt(pi) sum q^2.  Here each atom owns its full
-// row (one wavefront per atom), so the reference's i<j scatter becomes a
+// row (16 lanes per atom), so the reference's i<j scatter becomes a
 // gather with the 1/2 of the directed double count -- no atomics.
 //
 // Reciprocal space (Ewald class): the direct structure-factor sum over the half
@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "agpu_internal.hpp"
+#include "ewald_pair.hpp"
 #include "ewald_recip.hpp"
 #include "profile.hpp"
 
@@ -43,20 +44,6 @@ static void ewald_free(void *p) { delete static_cast<EwaldState *>(p); }
 // ---------------------------------------------------------------------------
 // real space
 // ---------------------------------------------------------------------------
-template <typename R> __device__ __forceinline__ R rerfc(R x);
-template <> __device__ __forceinline__ double rerfc<double>(double x) { return erfc(x); }
-template <> __device__ __forceinline__ float rerfc<float>(float x) { return erfcf(x); }
-template <typename R> __device__ __forceinline__ R rexp_(R x);
-template <> __device__ __forceinline__ double rexp_<double>(double x) { return exp(x); }
-template <> __device__ __forceinline__ float rexp_<float>(float x) { return expf(x); }
-
-template <typename T> __device__ __forceinline__ T wsum(T v)
-{
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
 // {x, y, z, q} per slot of the list's bin order (caller atom order[p])
 __global__ void k_ewald_pack(int nat, const SortedAtom *__restrict__ atoms, const int *__restrict__ order,
                              const double *__restrict__ q, double4 *__restrict__ q4)
@@ -67,15 +54,22 @@ __global__ void k_ewald_pack(int nat, const SortedAtom *__restrict__ atoms, cons
     q4[p] = make_double4(a.x, a.y, a.z, q[order[p]]);
 }
 
-template <typename R>
+constexpr int EW_NOSHIFT = (512 << 20) | (512 << 10) | 512;   // dc_pack(0, 0, 0)
+
+// EWG lanes per ion.  16 (four ions per wavefront) when the ions fill the
+// chip: with a wavefront per ion the ten sums over the lanes cost as much as
+// one of the three trips that 190 neighbours take.  216 000 ions: 560 -> 332 us
+// with 16 lanes and the shared exp of ewp_pair; 1200 ions: 12 us with 64
+// lanes, 17 with 16.
+template <typename R, int EWG>
 __global__ void __launch_bounds__(256)
 k_ewald_real(int nat, const int *__restrict__ order, const double4 *__restrict__ q4, CellArg C, NlRows L,
              double cutoff_sq, double beta, double sqrt_alpha_pi, double *__restrict__ f, double *__restrict__ phi,
              double *__restrict__ partial)
 {
-    __shared__ double s_red[4][10];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ai = blockIdx.x * 4 + wave;
+    __shared__ double s_red[4][7];
+    const int lane = threadIdx.x & (EWG - 1), wave = threadIdx.x >> 6;
+    const int ai = xcd_block() * (256 / EWG) + threadIdx.x / EWG;
     double e = 0.0, acc[3] = {0, 0, 0}, ph = 0.0;
     double w[6] = {0, 0, 0, 0, 0, 0};
     int i = -1;
@@ -88,61 +82,60 @@ k_ewald_real(int nat, const int *__restrict__ order, const double4 *__restrict__
             const double ri[3] = {hi.x, hi.y, hi.z};
             int n;
             const int2 *row = nl_row(L, ai, n);
-            const R b = (R)beta, sap = (R)sqrt_alpha_pi, al = (R)(beta * beta);
-            for (int s = lane; s < n; s += 64) {
-                int2 en = row[s];
+            const R b = (R)beta, sap = (R)sqrt_alpha_pi;
+            for (int s = lane; s < n; s += EWG) {
+                const int2 en = row[s];
                 const double4 qa = q4[en.x];
                 const double qj = qa.w;
                 if (!(fabs(qj) > 1e-10)) continue;
-                int a, bb, c;
-                dc_unpack(en.y, a, bb, c);
-                const double rj[3] = {qa.x, qa.y, qa.z};
-                double d[3];
-                delta_r(C, ri, rj, a, bb, c, d);
-                double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+                double d[3] = {ri[0] - qa.x, ri[1] - qa.y, ri[2] - qa.z};
+                if (en.y != EW_NOSHIFT) {
+                    int a, bb, c;
+                    dc_unpack(en.y, a, bb, c);
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) d[x] += image_x(C, x, a, bb, c);
+                }
+                const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
                 if (!(r2 < cutoff_sq)) continue;
-                double ar = sqrt(r2);
-                R arr = (R)ar;
-                R ec = rerfc<R>(b * arr);
-                R rinv = (R)1 / arr;
-                R hlp1 = ec * rinv;
-                R fr = rinv * rinv * rinv * (ec + (R)2 * sap * arr * rexp_<R>(-al * (R)r2));
-                double qq = qi * qj;
-                e += 0.5 * qq * (double)hlp1;
-                ph += qj * (double)hlp1;
-                double fs = qq * (double)fr;
-                double h[3] = {fs * d[0], fs * d[1], fs * d[2]};
+                double hlp1, fr;
+                ewp_pair(r2, b, sap, hlp1, fr);
+                ph += qj * hlp1;
+                const double fs = qj * fr;
+                const double h[3] = {fs * d[0], fs * d[1], fs * d[2]};
                 acc[0] += h[0];
                 acc[1] += h[1];
                 acc[2] += h[2];
-                w[0] -= 0.5 * d[0] * h[0];
-                w[1] -= 0.5 * d[1] * h[1];
-                w[2] -= 0.5 * d[2] * h[2];
-                w[3] -= 0.5 * d[1] * h[2];
-                w[4] -= 0.5 * d[0] * h[2];
-                w[5] -= 0.5 * d[0] * h[1];
+                w[0] += d[0] * h[0];
+                w[1] += d[1] * h[1];
+                w[2] += d[2] * h[2];
+                w[3] += d[1] * h[2];
+                w[4] += d[0] * h[2];
+                w[5] += d[0] * h[1];
             }
         }
     }
-    e = wsum(e);
-    ph = wsum(ph);
-    for (int x = 0; x < 3; ++x) acc[x] = wsum(acc[x]);
-    for (int k = 0; k < 6; ++k) w[k] = wsum(w[k]);
+    ph = group_sum<EWG>(ph);
+    for (int x = 0; x < 3; ++x) acc[x] = group_sum<EWG>(acc[x]);
     if (i >= 0 && lane == 0) {
+        e = 0.5 * qi * ph;
         // self term (pme.f90:467-472; phi: pme.f90:256)
         if (fabs(qi) > 1e-10) ph -= 2.0 * qi * sqrt_alpha_pi;
         e -= qi * qi * sqrt_alpha_pi;
         if (f) {
-            f[3 * (size_t)i] += acc[0];
-            f[3 * (size_t)i + 1] += acc[1];
-            f[3 * (size_t)i + 2] += acc[2];
+            f[3 * (size_t)i] += qi * acc[0];
+            f[3 * (size_t)i + 1] += qi * acc[1];
+            f[3 * (size_t)i + 2] += qi * acc[2];
         }
         if (phi) phi[i] += ph;
     }
-    if (lane == 0) {
-        s_red[wave][0] = e;
-        for (int k = 0; k < 6; ++k) s_red[wave][1 + k] = w[k];
-    }
+    // the wavefront's sums of the energy and of -1/2 q_i d x h over its ions
+    double v[7] = {e, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[1 + k] = -0.5 * qi * w[k];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) v[k] = group_sum<64>(v[k]);
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 7; ++k) s_red[wave][k] = v[k];
     __syncthreads();
     if (threadIdx.x < 7) {
         int qn = threadIdx.x;
@@ -198,7 +191,8 @@ static int ewald_run(agpu_potential *pot, const double *q, double *epot, double 
     CellArg C;
     std::memcpy(C.A, p->cell.A, sizeof C.A);
     const double sap = std::sqrt(st->beta * st->beta / M_PI);
-    const int nblk_r = (nat + 3) / 4;
+    const bool few = nat < 16384;       // fewer than four wavefronts per SIMD with 16 lanes each
+    const int ipb = few ? 4 : 16, nblk_r = (nat + ipb - 1) / ipb;
     const int nrec_k = st->pme ? 0 : st->recip.ntile;
     AGPU_CHECK(st->partial.reserve(sizeof(double) * 10 * (size_t)(nblk_r + nrec_k + 1)));
     double *part = st->partial.as<double>();
@@ -208,11 +202,11 @@ static int ewald_run(agpu_potential *pot, const double *q, double *epot, double 
     double4 *q4 = st->q4.as<double4>();
     AGPU_LAUNCH("ewald_pack", k_ewald_pack, dim3((nat + 255) / 256), dim3(256), 0, s, nat, L.atoms, order, q, q4);
     if (pot->precision == AGPU_PREC_MIXED)
-        AGPU_LAUNCH("ewald_real_mixed", k_ewald_real<float>, dim3(nblk_r), dim3(256), 0, s, nat, order, q4, C, L,
-                    st->cutoff * st->cutoff, st->beta, sap, f, phi, part);
+        AGPU_LAUNCH("ewald_real_mixed", (few ? k_ewald_real<float, 64> : k_ewald_real<float, 16>), dim3(nblk_r),
+                    dim3(256), 0, s, nat, order, q4, C, L, st->cutoff * st->cutoff, st->beta, sap, f, phi, part);
     else
-        AGPU_LAUNCH("ewald_real_fp64", k_ewald_real<double>, dim3(nblk_r), dim3(256), 0, s, nat, order, q4, C, L,
-                    st->cutoff * st->cutoff, st->beta, sap, f, phi, part);
+        AGPU_LAUNCH("ewald_real_fp64", (few ? k_ewald_real<double, 64> : k_ewald_real<double, 16>), dim3(nblk_r),
+                    dim3(256), 0, s, nat, order, q4, C, L, st->cutoff * st->cutoff, st->beta, sap, f, phi, part);
     if (st->pme) {
         // reciprocal record after the real-space block records
         AGPU_CHECK(pme_recip(st->pme, p, q, st->beta, part + 10 * (size_t)nblk_r, f, phi));

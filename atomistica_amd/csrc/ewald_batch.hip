@@ -5,12 +5,11 @@
 // real space and self term of pme.f90:215-321, 386-437, 467-472; reciprocal
 // space as the direct structure-factor sum over the half space of
 // k = 2 pi Bbox^T n, |k| <= kmax, in ewald_recip.hip):
-//   k_ewb_real<R>  one wavefront per tile of <= 64 ions of one structure:
-//                  every ion of the structure is staged through LDS and every
-//                  periodic image within the cut-off is summed (the image
-//                  range per axis comes from the reciprocal vectors), so no
-//                  neighbour list is stored.  erfc/exp in R (double, or float
-//                  with FP64 distances and FP64 accumulation).
+//   k_ewb_real<R>  one wavefront per ion: every ion of the structure and its
+//                  images are screened in FP32, those within r_c collected
+//                  in LDS and summed, so no neighbour list is stored.  erfc
+//                  and exp in R (double, or float with FP64 distances and
+//                  FP64 accumulation).
 //   k_ewb_sum      one wavefront per structure: energy and virial from the
 //                  per-ion records and those of the reciprocal sum in a
 //                  fixed order.
@@ -22,23 +21,17 @@
 
 #include "agpu_internal.hpp"
 #include "batch_internal.hpp"
+#include "ewald_pair.hpp"
 #include "ewald_recip.hpp"
 #include "profile.hpp"
 
 namespace agpu {
 
-constexpr int EWB_T = 64;      // ions per wavefront tile
-
-struct EwbTile {
-    int s, b, e, pad;      // structure, [b, e): ions
-};
-
 struct EwbState {
     double kmax = 0.0;
     uint64_t struct_rev = ~0ull;
-    std::vector<EwbTile> itiles;
     EwrState recip;
-    DevBuf d_itiles, d_ionrec, d_krec, d_q;
+    DevBuf d_u, d_ionrec, d_krec, d_q;
 };
 
 static void ewb_free(void *p) { delete static_cast<EwbState *>(p); }
@@ -46,124 +39,183 @@ static void ewb_free(void *p) { delete static_cast<EwbState *>(p); }
 // record layout (7 doubles): e, w_xx, w_yy, w_zz, w_yz, w_xz, w_xy
 constexpr int EWB_REC = 7;
 
-template <typename R> __device__ __forceinline__ R ewb_erfc(R x);
-template <> __device__ __forceinline__ double ewb_erfc<double>(double x) { return erfc(x); }
-template <> __device__ __forceinline__ float ewb_erfc<float>(float x) { return erfcf(x); }
-template <typename R> __device__ __forceinline__ R ewb_exp(R x);
-template <> __device__ __forceinline__ double ewb_exp<double>(double x) { return exp(x); }
-template <> __device__ __forceinline__ float ewb_exp<float>(float x) { return expf(x); }
-
 struct EwbGeom {
     const int *off;        // atom offsets per structure
     const double *cell;    // 9 per structure, cell[3k+x] = a_k[x]
     const double *rec;     // 9 per structure, rec[3k+x] = b_k[x], a_k . b_l = delta_kl
 };
 
+// Fractional coordinates per ion in units of 2^-32 of a lattice vector: the
+// difference of two, taken modulo 2^32 as a signed number, is the difference
+// to the nearest image along each axis.
+__global__ void k_ewb_frac(int n, const int *__restrict__ sof, const double *__restrict__ rec,
+                           const double *__restrict__ r, int4 *__restrict__ u)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const double *b = rec + 9 * (size_t)sof[j];
+    const double x = r[3 * (size_t)j], y = r[3 * (size_t)j + 1], z = r[3 * (size_t)j + 2];
+    int v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        double s = b[3 * k] * x + b[3 * k + 1] * y + b[3 * k + 2] * z;
+        s -= floor(s);
+        v[k] = (int)(unsigned)(long long)(s * 4294967296.0);
+    }
+    u[j] = make_int4(v[0], v[1], v[2], 0);
+}
+
+// A wavefront per ion.  The lanes screen 64 ions of the structure at a time
+// in FP32 (with slack for the rounding), for the nearest image and, in cells
+// below twice the cut-off, the images around it; those that pass are
+// collected in LDS and evaluated 64 at a time.  A lane per ion that walked
+// all candidates by itself ran the pair evaluation for nearly every
+// candidate, since one of 64 ions nearly always had it inside the cut-off.
+constexpr int EWB_W = 4;            // wavefronts per workgroup
+constexpr int EWB_C = 4;            // candidates per lane loaded together
+
 template <typename R>
-__global__ void __launch_bounds__(EWB_T)
-k_ewb_real(const EwbTile *__restrict__ tiles, EwbGeom G, const double *__restrict__ r,
+__global__ void __launch_bounds__(64 * EWB_W)
+k_ewb_real(int n, const int *__restrict__ sof, EwbGeom G, const double *__restrict__ r, const int4 *__restrict__ u,
            const double *__restrict__ q, double cutoff, double beta, double *__restrict__ f,
            double *__restrict__ phi, double *__restrict__ ionrec)
 {
-    __shared__ double sh_r[EWB_T][3];
-    __shared__ double sh_q[EWB_T];
-    const EwbTile T = tiles[blockIdx.x];
-    const int lane = threadIdx.x;
-    const int i = T.b + lane;
-    const bool act = i < T.e;
-    double A[9], b[9], t[3];
+    __shared__ int2 queue[EWB_W][64 * (EWB_C + 1)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * EWB_W + wave;
+    if (i >= n) return;
+    const int st = sof[i];
+    int2 *Q = queue[wave];
+    double A[9], b[9];
+    int m[3];
+    float Af[9], reach = 0.f;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-        A[k] = G.cell[9 * (size_t)T.s + k];
-        b[k] = G.rec[9 * (size_t)T.s + k];
+        A[k] = G.cell[9 * (size_t)st + k];
+        b[k] = G.rec[9 * (size_t)st + k];
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-        t[k] = cutoff * sqrt(b[3 * k] * b[3 * k] + b[3 * k + 1] * b[3 * k + 1] + b[3 * k + 2] * b[3 * k + 2]);
+    for (int k = 0; k < 3; ++k) {
+        const double t =
+            cutoff * sqrt(b[3 * k] * b[3 * k] + b[3 * k + 1] * b[3 * k + 1] + b[3 * k + 2] * b[3 * k + 2]);
+        // images around the nearest one that can come within the cut-off
+        m[k] = max(0, (int)ceil(t - 0.5 + 1e-6));
+        const float len = (float)sqrt(A[3 * k] * A[3 * k] + A[3 * k + 1] * A[3 * k + 1] + A[3 * k + 2] * A[3 * k + 2]);
+        reach += (0.5f + m[k]) * len;
+#pragma unroll
+        for (int x = 0; x < 3; ++x) Af[3 * k + x] = (float)(A[3 * k + x]);
+    }
     const double rc2 = cutoff * cutoff;
+    // FP32 rounding of a difference vector: a few 2^-24 of its summands
+    const float rs = (float)cutoff * 1.000001f + 1e-6f * reach, rs2 = rs * rs;
     const double sap = beta / sqrt(M_PI);
-    const R bR = (R)beta, sapR = (R)sap, alR = (R)(beta * beta);
-    double ri[3] = {0.0, 0.0, 0.0}, qi = 0.0;
-    if (act) {
-        ri[0] = r[3 * (size_t)i];
-        ri[1] = r[3 * (size_t)i + 1];
-        ri[2] = r[3 * (size_t)i + 2];
-        qi = q[i];
-    }
-    const bool live = act && fabs(qi) > 1e-10;
-    double e = 0.0, ph = 0.0, acc[3] = {0.0, 0.0, 0.0}, w[6] = {0, 0, 0, 0, 0, 0};
-    const int a0 = G.off[T.s], a1 = G.off[T.s + 1];
-    for (int base = a0; base < a1; base += EWB_T) {
-        const int jj = base + lane;
-        __syncthreads();
-        if (jj < a1) {
-            sh_r[lane][0] = r[3 * (size_t)jj];
-            sh_r[lane][1] = r[3 * (size_t)jj + 1];
-            sh_r[lane][2] = r[3 * (size_t)jj + 2];
-            sh_q[lane] = q[jj];
-        }
-        __syncthreads();
-        if (!live) continue;
-        const int m = min(EWB_T, a1 - base);
-        for (int tt = 0; tt < m; ++tt) {
-            const double qj = sh_q[tt];
-            if (!(fabs(qj) > 1e-10)) continue;
-            const int j = base + tt;
-            const double d0[3] = {ri[0] - sh_r[tt][0], ri[1] - sh_r[tt][1], ri[2] - sh_r[tt][2]};
-            int lo[3], hi[3];
+    const double ri[3] = {r[3 * (size_t)i], r[3 * (size_t)i + 1], r[3 * (size_t)i + 2]};
+    const double qi = q[i];
+    const int4 ui = u[i];
+    double ph = 0.0, acc[3] = {0.0, 0.0, 0.0}, w[6] = {0, 0, 0, 0, 0, 0};
+    const int a0 = G.off[st], a1 = G.off[st + 1];
+
+    // evaluates the collected candidates from .. from + cnt - 1, one per lane
+    auto evaluate = [&](int from, int cnt) {
+        if (lane >= cnt) return;
+        const int2 c = Q[from + lane];
+        const int j = c.x;
+        const double qj = q[j];
+        if (!(fabs(qj) > 1e-10)) return;
+        const int4 uj = u[j];
+        const double d0[3] = {ri[0] - r[3 * (size_t)j], ri[1] - r[3 * (size_t)j + 1], ri[2] - r[3 * (size_t)j + 2]};
+        const int du[3] = {(int)((unsigned)ui.x - (unsigned)uj.x), (int)((unsigned)ui.y - (unsigned)uj.y),
+                           (int)((unsigned)ui.z - (unsigned)uj.z)};
+        double nk[3];
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const double ds = b[3 * k] * d0[0] + b[3 * k + 1] * d0[1] + b[3 * k + 2] * d0[2];
-                lo[k] = (int)ceil(-ds - t[k] - 1e-9);
-                hi[k] = (int)floor(-ds + t[k] + 1e-9);
+        for (int k = 0; k < 3; ++k) {
+            // the whole turns between the difference and its wrapped form
+            const double ds = b[3 * k] * d0[0] + b[3 * k + 1] * d0[1] + b[3 * k + 2] * d0[2];
+            nk[k] = rint((double)du[k] * 2.3283064365386963e-10 - ds) + (double)(((c.y >> (10 * k)) & 1023) - 512);
+        }
+        if (j == i && nk[0] == 0.0 && nk[1] == 0.0 && nk[2] == 0.0) return;
+        double d[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) d[x] = d0[x] + (A[x] * nk[0] + A[3 + x] * nk[1] + A[6 + x] * nk[2]);
+        const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        if (!(r2 < rc2)) return;
+        double hlp, fr;
+        ewp_pair(r2, (R)beta, (R)sap, hlp, fr);
+        ph += qj * hlp;
+        const double fs = qj * fr;
+        const double h[3] = {fs * d[0], fs * d[1], fs * d[2]};
+        acc[0] += h[0];
+        acc[1] += h[1];
+        acc[2] += h[2];
+        w[0] += d[0] * h[0];
+        w[1] += d[1] * h[1];
+        w[2] += d[2] * h[2];
+        w[3] += d[1] * h[2];
+        w[4] += d[0] * h[2];
+        w[5] += d[0] * h[1];
+    };
+
+    if (fabs(qi) > 1e-10) {
+        const int w0 = 2 * m[0] + 1, w1 = 2 * m[1] + 1, w2 = 2 * m[2] + 1, ncomb = w0 * w1 * w2;
+        int nq = 0;
+        for (int base = a0; base < a1; base += 64 * EWB_C) {
+            float du[EWB_C][3];
+            int4 uj[EWB_C];
+#pragma unroll
+            for (int c = 0; c < EWB_C; ++c) uj[c] = u[min(base + 64 * c + lane, a1 - 1)];
+#pragma unroll
+            for (int c = 0; c < EWB_C; ++c) {
+                du[c][0] = (float)(int)((unsigned)ui.x - (unsigned)uj[c].x) * 2.3283064e-10f;
+                du[c][1] = (float)(int)((unsigned)ui.y - (unsigned)uj[c].y) * 2.3283064e-10f;
+                du[c][2] = (float)(int)((unsigned)ui.z - (unsigned)uj[c].z) * 2.3283064e-10f;
             }
-            for (int n0 = lo[0]; n0 <= hi[0]; ++n0)
-                for (int n1 = lo[1]; n1 <= hi[1]; ++n1)
-                    for (int n2 = lo[2]; n2 <= hi[2]; ++n2) {
-                        if (j == i && n0 == 0 && n1 == 0 && n2 == 0) continue;
-                        double d[3];
+            for (int o = 0; o < ncomb; ++o) {
+                const int n0 = o / (w1 * w2) - m[0], n1 = (o / w2) % w1 - m[1], n2 = o % w2 - m[2];
+                const float f0 = (float)n0, f1 = (float)n1, f2 = (float)n2;
+                const int code = (n0 + 512) | ((n1 + 512) << 10) | ((n2 + 512) << 20);
 #pragma unroll
-                        for (int x = 0; x < 3; ++x)
-                            d[x] = d0[x] + (A[x] * n0 + A[3 + x] * n1 + A[6 + x] * n2);
-                        const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-                        if (!(r2 < rc2)) continue;
-                        const double ar = sqrt(r2);
-                        const R arr = (R)ar;
-                        const R ec = ewb_erfc<R>(bR * arr);
-                        const R rinv = (R)1 / arr;
-                        const R hlp = ec * rinv;
-                        const R fr = rinv * rinv * rinv * (ec + (R)2 * sapR * arr * ewb_exp<R>(-alR * (R)r2));
-                        const double qq = qi * qj;
-                        e += 0.5 * qq * (double)hlp;
-                        ph += qj * (double)hlp;
-                        const double fs = qq * (double)fr;
-                        const double h[3] = {fs * d[0], fs * d[1], fs * d[2]};
-                        acc[0] += h[0];
-                        acc[1] += h[1];
-                        acc[2] += h[2];
-                        w[0] -= 0.5 * d[0] * h[0];
-                        w[1] -= 0.5 * d[1] * h[1];
-                        w[2] -= 0.5 * d[2] * h[2];
-                        w[3] -= 0.5 * d[1] * h[2];
-                        w[4] -= 0.5 * d[0] * h[2];
-                        w[5] -= 0.5 * d[0] * h[1];
-                    }
+                for (int c = 0; c < EWB_C; ++c) {
+                    const float v0 = du[c][0] + f0, v1 = du[c][1] + f1, v2 = du[c][2] + f2;
+                    const float x = Af[0] * v0 + Af[3] * v1 + Af[6] * v2;
+                    const float y = Af[1] * v0 + Af[4] * v1 + Af[7] * v2;
+                    const float z = Af[2] * v0 + Af[5] * v1 + Af[8] * v2;
+                    const int j = base + 64 * c + lane;
+                    const bool in = j < a1 && x * x + y * y + z * z < rs2;
+                    const unsigned long long mk = __ballot(in);
+                    if (in)
+                        Q[nq + __builtin_amdgcn_mbcnt_hi((unsigned)(mk >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((unsigned)mk, 0))] = make_int2(j, code);
+                    nq += __popcll(mk);
+                }
+                // the last ones collected go first: nothing is moved
+                const bool last = base + 64 * EWB_C >= a1 && o == ncomb - 1;
+                while (nq >= 64 || (last && nq > 0)) {
+                    const int cnt = min(nq, 64);
+                    __builtin_amdgcn_wave_barrier();
+                    evaluate(nq - cnt, cnt);
+                    __builtin_amdgcn_wave_barrier();
+                    nq -= cnt;
+                }
+            }
         }
     }
-    if (!act) return;
-    // self term (pme.f90:467-472; phi: pme.f90:256)
-    if (live) ph -= 2.0 * qi * sap;
-    e -= qi * qi * sap;
-    if (f) {
-        f[3 * (size_t)i] += acc[0];
-        f[3 * (size_t)i + 1] += acc[1];
-        f[3 * (size_t)i + 2] += acc[2];
-    }
-    if (phi) phi[i] += ph;
-    double *rec = ionrec + EWB_REC * (size_t)i;
-    rec[0] = e;
+    ph = group_sum<64>(ph);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) rec[1 + k] = w[k];
+    for (int x = 0; x < 3; ++x) acc[x] = group_sum<64>(acc[x]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) w[k] = group_sum<64>(w[k]);
+    if (lane != 0) return;
+    double *o = ionrec + EWB_REC * (size_t)i;
+    // self term (pme.f90:467-472; phi: pme.f90:256)
+    o[0] = 0.5 * qi * ph - qi * qi * sap;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) o[1 + k] = -0.5 * qi * w[k];
+    if (f) {
+        f[3 * (size_t)i] += qi * acc[0];
+        f[3 * (size_t)i + 1] += qi * acc[1];
+        f[3 * (size_t)i + 2] += qi * acc[2];
+    }
+    if (phi) phi[i] += fabs(qi) > 1e-10 ? ph - 2.0 * qi * sap : ph;
 }
 
 // energy and virial per structure: one wavefront per structure, lane-strided
@@ -207,21 +259,6 @@ k_ewb_sum(int nstruct, const int *__restrict__ off, const int *__restrict__ tile
     }
 }
 
-static int ewb_ion_tiles(agpu_batch *b, EwbState &st)
-{
-    st.itiles.clear();
-    for (int s = 0; s < b->nstruct; ++s)
-        for (int a = b->h_off[s]; a < b->h_off[s + 1]; a += EWB_T)
-            st.itiles.push_back(EwbTile{s, a, std::min(a + EWB_T, b->h_off[s + 1]), 0});
-    AGPU_CHECK(st.d_itiles.reserve(sizeof(EwbTile) * (st.itiles.size() + 1)));
-    hipStream_t hs = stream();
-    if (!st.itiles.empty())
-        AGPU_HIP(hipMemcpyAsync(st.d_itiles.ptr, st.itiles.data(), sizeof(EwbTile) * st.itiles.size(),
-                                hipMemcpyHostToDevice, hs));
-    AGPU_HIP(hipStreamSynchronize(hs));
-    return AGPU_OK;
-}
-
 }  // namespace agpu
 
 using namespace agpu;
@@ -247,7 +284,6 @@ extern "C" int agpu_ewald_batch_compute(agpu_batch *b, const double *q, double c
         st.struct_rev = ~0ull;
         st.kmax = kmax;
         AGPU_CHECK(ewr_plan(st.recip, ns, b->h_cell.data(), b->h_off.data(), kmax));
-        AGPU_CHECK(ewb_ion_tiles(b, st));
         st.struct_rev = b->struct_rev;
     }
     hipStream_t s = stream();
@@ -270,16 +306,18 @@ extern "C" int agpu_ewald_batch_compute(agpu_batch *b, const double *q, double c
     AGPU_CHECK(st.d_ionrec.reserve(sizeof(double) * EWB_REC * ((size_t)n + 1)));
     AGPU_CHECK(st.d_krec.reserve(sizeof(double) * 10 * ((size_t)st.recip.ntile + 1)));
     EwbGeom G{b->off.as<int>(), b->cell.as<double>(), b->rec.as<double>()};
-    const int nit = (int)st.itiles.size();
-    if (nit > 0) {
+    if (n > 0) {
+        AGPU_CHECK(st.d_u.reserve(sizeof(int4) * (size_t)n));
+        int4 *u = st.d_u.as<int4>();
+        AGPU_LAUNCH("ewald_batch_frac", k_ewb_frac, dim3((n + 255) / 256), dim3(256), 0, s, n, b->sof.as<int>(),
+                    b->rec.as<double>(), b->r.as<double>(), u);
+        const dim3 g((n + EWB_W - 1) / EWB_W), t(64 * EWB_W);
         if (precision == AGPU_PREC_MIXED)
-            AGPU_LAUNCH("ewald_batch_real_mixed", k_ewb_real<float>, dim3(nit), dim3(EWB_T), 0, s,
-                        st.d_itiles.as<EwbTile>(), G, b->r.as<double>(), qv, cutoff, beta, fv, pv,
-                        st.d_ionrec.as<double>());
+            AGPU_LAUNCH("ewald_batch_real_mixed", k_ewb_real<float>, g, t, 0, s, n, b->sof.as<int>(), G,
+                        b->r.as<double>(), u, qv, cutoff, beta, fv, pv, st.d_ionrec.as<double>());
         else
-            AGPU_LAUNCH("ewald_batch_real_fp64", k_ewb_real<double>, dim3(nit), dim3(EWB_T), 0, s,
-                        st.d_itiles.as<EwbTile>(), G, b->r.as<double>(), qv, cutoff, beta, fv, pv,
-                        st.d_ionrec.as<double>());
+            AGPU_LAUNCH("ewald_batch_real_fp64", k_ewb_real<double>, g, t, 0, s, n, b->sof.as<int>(), G,
+                        b->r.as<double>(), u, qv, cutoff, beta, fv, pv, st.d_ionrec.as<double>());
     }
     AGPU_CHECK(ewr_run(st.recip, n, b->r.as<double>(), qv, b->sof.as<int>(), kmax, beta, st.d_krec.as<double>(), fv,
                        pv));

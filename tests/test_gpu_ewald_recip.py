@@ -120,3 +120,38 @@ def test_recip_forces_against_80_bit_sums():
     err = float(np.sqrt(((f - ref) ** 2).sum() / (ref ** 2).sum()))
     print("ewald forces, 512 ions: relative error against 80-bit sums %.2e" % err, flush=True)
     assert err < 5e-14
+
+
+@pytest.mark.parametrize("precision,rel", [("fp64", 1e-10), ("mixed", 2e-6)])
+@pytest.mark.parametrize("n,beta", [(1, 0.4), (15, 0.4), (17, 0.05), (65, 2.5), (700, 0.4), (17000, 0.4)])
+def test_real_space_ranges(n, beta, precision, rel):
+    """Real space alone (no k inside kmax): ions around the 16 and 64 lanes,
+    both lane widths, and beta r from 1e-3 to 10 (pairs as close as 0.02 A,
+    erfc down to 1e-45).  FP32 arithmetic: erfcf, expf and a division each
+    within a few 2^-24 of their term."""
+    from atomistica_amd import native as N
+    from atomistica_amd.batch import Batch, ewald_batch
+    rng = np.random.default_rng(n)
+    cell = _cell((9.0 + n ** (1 / 3.0),) * 3, 0.2)
+    pos, q = _ions(n, cell, 17 * n)
+    if n > 1:
+        pos[1] = pos[0] + np.array([0.02, 0.0, 0.0])
+    print("ewald real space: %d ions beta %g %s" % (n, beta, precision), flush=True)
+    p = N.from_atoms(pos, cell, [True] * 3, np.full(n, 11, np.int32))
+    nl = N.Neighbors(2000)
+    pot = N.Ewald(cutoff=RC, beta=beta, kmax=1e-3)
+    pot.set_precision(precision)
+    pot.bind_to(p, nl)
+    e, f, w = pot.energy_and_forces(p, nl, q)
+    re_, rf, rw, rp = O.ewald_real(pos, q, cell, O.nl_build(pos, cell, [True] * 3, RC, avgn=2000), RC, beta)
+    scale = np.abs(rf).max()
+    assert abs(e - re_) <= rel * max(1.0, np.abs(q * rp).sum())
+    assert np.abs(f - rf).max() <= rel * max(1.0, scale)
+    assert np.abs(w - rw).max() <= rel * max(1.0, np.abs(rw).max(), np.abs(q * rp).sum())
+    if n <= 700:
+        eb, fb, wb, pb = (t.cpu().numpy() for t in
+                          ewald_batch(Batch([(pos, cell)]), q, RC, beta, 1e-3, precision, phi=True))
+        assert abs(eb[0] - re_) <= rel * max(1.0, np.abs(q * rp).sum())
+        assert np.abs(fb - rf).max() <= rel * max(1.0, scale)
+        assert np.abs(wb[0] - rw).max() <= rel * max(1.0, np.abs(rw).max(), np.abs(q * rp).sum())
+        assert np.abs(pb - rp).max() <= rel * max(1.0, np.abs(rp).max())
