@@ -282,6 +282,15 @@ __device__ __forceinline__ int xcd_block()
     return (b % 8) * per + b / 8;
 }
 
+// LDS exchange inside one wavefront: what its lanes wrote is seen by its
+// lanes afterwards (LDS operations of a wavefront are carried out in order,
+// so this orders the compiler only)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // warp-level (wave64) helpers
 template <typename T> __device__ __forceinline__ T shfl_xor(T v, int m)
 {

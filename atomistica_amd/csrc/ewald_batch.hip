@@ -191,9 +191,9 @@ k_ewb_real(int n, const int *__restrict__ sof, EwbGeom G, const double *__restri
                 const bool last = base + 64 * EWB_C >= a1 && o == ncomb - 1;
                 while (nq >= 64 || (last && nq > 0)) {
                     const int cnt = min(nq, 64);
-                    __builtin_amdgcn_wave_barrier();
+                    wave_sync();
                     evaluate(nq - cnt, cnt);
-                    __builtin_amdgcn_wave_barrier();
+                    wave_sync();
                     nq -= cnt;
                 }
             }

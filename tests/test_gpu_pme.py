@@ -89,3 +89,32 @@ def test_pme_reproducible_and_charge_derivative():
     qm[3] -= h
     d = (gpu(pos, qp, cell, pbc, Z, 5.0, (10, 12, 14), 8)[0] - gpu(pos, qm, cell, pbc, Z, 5.0, (10, 12, 14), 8)[0]) / (2 * h)
     assert abs(d - a[3][3]) < 1e-7
+
+
+EDGES = [(n, grid, order) for n in (2, 5) for grid, order in
+         [((3, 3, 3), 3), ((4, 7, 9), 4), ((8, 8, 8), 5), ((9, 16, 17), 6), ((7, 24, 8), 7), ((8, 9, 31), 8),
+          ((9, 9, 9), 9), ((10, 12, 23), 10), ((11, 24, 12), 11), ((12, 13, 40), 12)]] + [(900, (16, 9, 25), 8)]
+
+
+@pytest.mark.parametrize("n,grid,order", EDGES)
+@pytest.mark.parametrize("shear", [0.0, 0.15])
+def test_pme_brick_edges(n, grid, order, shear):
+    """Grids around the 8^3 cells of a brick, down to the order itself (a
+    brick's points then cover the grid more than once), every order, odd and
+    even lengths (the Nyquist terms of a sheared cell), few ions and many in
+    one brick, ions outside the cell."""
+    rng = np.random.default_rng(n + order)
+    # symmetric strain: the reference's reciprocal indexing then holds
+    m = np.eye(3) + shear * np.array([[0, 1, 0.5], [1, 0, -0.4], [0.5, -0.4, 0]])
+    cell = np.diag([9.0, 10.0, 12.0]) @ m
+    pos = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))) @ cell
+    q = rng.normal(size=n)
+    # neutral: the m = 0 term, left in place as the reference does, then adds
+    # nothing, while the oracle drops it
+    q -= q.mean()
+    Z = np.full(n, 11, np.int32)
+    print("pme edges", n, grid, order, shear, flush=True)
+    e0, f0, w0, p0 = oracle(pos, q, cell, [True] * 3, 4.0, grid, order)
+    e, f, w, phi = gpu(pos, q, cell, [True] * 3, Z, 4.0, grid, order)
+    assert abs(e - e0) <= REL * max(1.0, abs(e0))
+    assert close(f, f0) and close(w, w0) and close(phi, p0)
