@@ -218,6 +218,7 @@ __global__ void k_gather(int nat, const double *__restrict__ r, BinGeom g, CellA
 constexpr int NL_R = 4;         // candidate slots per lane (registers): 256 per pass
 constexpr int NL_WAVES = 4;     // wavefronts per block
 constexpr int NL_HMAX = 64;     // home atoms per pass
+constexpr int NL_Q = 64 * NL_R; // candidates collected for a pass
 
 // smallest b in [0, 64) with pre[b] > e (pre = inclusive prefix, pre[63] > e)
 __device__ __forceinline__ int find_bin(const int *pre, int e)
@@ -246,6 +247,13 @@ __device__ __forceinline__ int off_pack(int a, int b, int c) { return ((a + 128)
 struct NlShared {
     int hi[NL_HMAX], ho[NL_HMAX], hp[NL_HMAX];
     int pre[64], start[64], bu[64], boff[64];
+};
+
+template <bool CULL> struct NlQueue {
+    int src[NL_Q], bu[NL_Q], off[NL_Q];     // slot, bin shift and stencil offset
+};
+template <> struct NlQueue<false> {
+    int src[1], bu[1], off[1];
 };
 
 // pair shift s = w_home + u_bin - w_cand; distance as the reference writes it
@@ -311,14 +319,20 @@ __device__ __forceinline__ void row_stats_wave(int longest, int last, int2 *__re
 // MULTI: blocks of B > 1 bins, whose candidates are checked against each home
 // atom's own stencil.  nsub wavefronts share a block's home atoms; a row is
 // one wavefront's, so the share does not change it.
-template <bool ORTHO, bool MULTI>
-__global__ void __launch_bounds__(256)
+// CULL: candidates that cannot reach the box around the wavefront's home atoms
+// are left out before the home atoms walk the rest, kept in their order.
+// Four wavefronts per SIMD without CULL (21 registers of the rare paths spill:
+// Cu 200 -> 178 us), three with it.
+template <bool ORTHO, bool MULTI, bool CULL>
+__global__ void __launch_bounds__(256, CULL ? 3 : 4)
 k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const SortedAtom *__restrict__ atoms,
             const int *__restrict__ cell_start, int *__restrict__ scnt,
             int2 *__restrict__ stage, int S, int *__restrict__ flags, int2 *__restrict__ part)
 {
     __shared__ NlShared sh[NL_WAVES];
+    __shared__ NlQueue<CULL> shq[NL_WAVES];
     NlShared &L = sh[threadIdx.x >> 6];
+    NlQueue<CULL> &Q = shq[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63;
     const int nbx = (g.nc[0] + B - 1) / B, nby = (g.nc[1] + B - 1) / B, nbz = (g.nc[2] + B - 1) / B;
     // wavefront sub of nsub takes its share of the block's home atoms
@@ -361,6 +375,7 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
     const int nst = sx * sy * sz;
     int wmax = 0, wlast = 0;
     bool stage_over = false, img_bad = false;
+    const double rc = sqrt(cutoff_sq);
 
     for (int a0 = M0; a0 < MH; a0 += NL_HMAX) {
         const int ma = min(NL_HMAX, MH - a0);
@@ -384,6 +399,32 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
         const int hp_lane = L.hp[lane];
         const int ho_lane = MULTI ? L.ho[lane] : 0;
         int hcnt_lane = 0;
+        // the home atoms' box, in the cell of their bins (r + A.w)
+        double hlo[3], hhi[3], hsize = 0.0;
+        if (CULL) {
+            double h[3] = {0.0, 0.0, 0.0};
+            if (lane < ma) {
+                const SortedAtom A = atoms[hp_lane];
+                int w0, w1, w2;
+                dc_unpack(A.w, w0, w1, w2);
+                h[0] = A.x + image_x(C, 0, w0, w1, w2);
+                h[1] = A.y + image_x(C, 1, w0, w1, w2);
+                h[2] = A.z + image_x(C, 2, w0, w1, w2);
+                hsize = fabs(A.x) + fabs(A.y) + fabs(A.z) + fabs(h[0]) + fabs(h[1]) + fabs(h[2]);
+            }
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) hsize = fmax(hsize, __shfl_xor(hsize, o, 64));
+#pragma unroll
+            for (int x = 0; x < 3; ++x) {
+                hlo[x] = lane < ma ? h[x] : __longlong_as_double(0x7ff0000000000000ll);
+                hhi[x] = lane < ma ? h[x] : -hlo[x];
+#pragma unroll
+                for (int o = 32; o >= 1; o >>= 1) {
+                    hlo[x] = fmin(hlo[x], __shfl_xor(hlo[x], o, 64));
+                    hhi[x] = fmax(hhi[x], __shfl_xor(hhi[x], o, 64));
+                }
+            }
+        }
 
         for (int st0 = 0; st0 < nst; st0 += 64) {
             // lane L owns stencil bin st0 + L of the block (x-major order)
@@ -426,33 +467,94 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
             L.boff[lane] = oL;
             __builtin_amdgcn_wave_barrier();
             const int T = L.pre[63];
-            for (int c0 = 0; c0 < T; c0 += 64 * NL_R) {
+            int nq = 0;
+            for (int e0 = 0; e0 < T; e0 += CULL ? 64 : NL_Q) {
+                int NC = min(NL_Q, T - e0);
+                if (CULL) {
+                    // ---- collect the candidates that can reach a home atom ----
+                    const int e = e0 + lane;
+                    int b = 0, src = 0;
+                    bool in = e < T;
+                    if (in) {
+                        b = find_bin(L.pre, e);
+                        src = L.start[b] + e - (b ? L.pre[b - 1] : 0);
+                        // its place in the home atoms' cell, r - A.(u - w), and
+                        // the distance from there to their box.  Places, box and
+                        // the FP64 test below round by a few 2^-53 of the
+                        // coordinates and shifts that enter; 1e-14 of them is
+                        // allowed.
+                        const SortedAtom A = atoms[src];
+                        int u0, u1, u2, w0, w1, w2;
+                        dc_unpack(L.bu[b], u0, u1, u2);
+                        dc_unpack(A.w, w0, w1, w2);
+                        const double q[3] = {A.x, A.y, A.z};
+                        double gap = 0.0, size = hsize;
+#pragma unroll
+                        for (int x = 0; x < 3; ++x) {
+                            const double c =
+                                q[x] - (ORTHO ? C.A[4 * x] * (double)(x == 0 ? u0 - w0 : x == 1 ? u1 - w1 : u2 - w2)
+                                              : image_x(C, x, u0 - w0, u1 - w1, u2 - w2));
+                            const double o = fmax(fmax(hlo[x] - c, c - hhi[x]), 0.0);
+                            gap = fma(o, o, gap);
+                            size += fabs(q[x]) + fabs(c);
+                        }
+                        const double reach = fma(1e-14, size, rc);
+                        in = !(gap > reach * reach);      // NaN counts as near
+                    }
+                    const unsigned long long m = __ballot(in);
+                    if (in) {
+                        const int at = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)nq));
+                        Q.src[at] = src;
+                        Q.bu[at] = L.bu[b];
+                        if (MULTI) Q.off[at] = L.boff[b];
+                    }
+                    nq += __popcll(m);
+                    // a full pass, or the last one of these bins
+                    if (nq <= NL_Q - 64 && e0 + 64 < T) continue;
+                    NC = nq;
+                    nq = 0;
+                    if (NC == 0) continue;
+                    wave_sync();
+                }
+                // slot, bin shift and stencil offset of candidate e of the pass
+                auto candidate = [&](int e, int &src, int &bu, int &off) {
+                    if (CULL) {
+                        src = Q.src[e];
+                        bu = Q.bu[e];
+                        off = MULTI ? Q.off[e] : 0;
+                    } else {
+                        const int b = find_bin(L.pre, e0 + e);
+                        src = L.start[b] + e0 + e - (b ? L.pre[b - 1] : 0);
+                        bu = L.bu[b];
+                        off = MULTI ? L.boff[b] : 0;
+                    }
+                };
                 // ---- load this pass's candidates into registers ----
                 double cx[NL_R], cy[NL_R], cz[NL_R], cp0[NL_R], cp1[NL_R], cp2[NL_R];
                 int cj[NL_R], co[NL_R], cpk[NL_R];
                 bool cv[NL_R];
 #pragma unroll
                 for (int r = 0; r < NL_R; ++r) {
-                    const int e = c0 + 64 * r + lane;
-                    cv[r] = e < T;
+                    const int e = 64 * r + lane;
+                    cv[r] = e < NC;
                     cx[r] = cy[r] = cz[r] = 0.0;
                     cp0[r] = cp1[r] = cp2[r] = 0.0;
                     cj[r] = -1;
                     co[r] = 0;
                     cpk[r] = -1;
                     if (cv[r]) {
-                        const int b = find_bin(L.pre, e);
-                        const int src = L.start[b] + e - (b ? L.pre[b - 1] : 0);
+                        int src, bu;
+                        candidate(e, src, bu, co[r]);
                         const SortedAtom A = atoms[src];
                         int u0, u1, u2, w0, w1, w2;
-                        dc_unpack(L.bu[b], u0, u1, u2);
+                        dc_unpack(bu, u0, u1, u2);
                         dc_unpack(A.w, w0, w1, w2);
                         cx[r] = A.x;
                         cy[r] = A.y;
                         cz[r] = A.z;
                         cj[r] = src;
                         const int t0 = u0 - w0, t1 = u1 - w1, t2 = u2 - w2;
-                        if (MULTI) co[r] = L.boff[b];
                         if (ORTHO) {
                             cp0[r] = C.A[0] * (double)t0;
                             cp1[r] = C.A[4] * (double)t1;
@@ -506,7 +608,7 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
                         // one exec region guards the store
 #pragma unroll
                         for (int r = 0; r < NL_R; ++r) {
-                            if (c0 + 64 * r >= T) break;     // slot row past the last candidate
+                            if (64 * r >= NC) break;         // slot row past the last candidate
                             const double d2 = pair_d2_pre(H.x, H.y, H.z, cx[r], cy[r], cz[r], cp0[r], cp1[r], cp2[r]);
                             const bool acc = (bool)((int)member(r) & (int)(d2 < cutoff_sq) &
                                                     (int)((cj[r] != hp) | (cpk[r] != DC_ZERO)));
@@ -520,17 +622,16 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
                     } else {
 #pragma unroll
                         for (int r = 0; r < NL_R; ++r) {
-                            if (c0 + 64 * r >= T) break;
+                            if (64 * r >= NC) break;
                             int t0 = 0, t1 = 0, t2 = 0;
                             if (cpk[r] >= 0) {
                                 dc_unpack(cpk[r], t0, t1, t2);
                             } else if (cv[r]) {
                                 // shift beyond the packed range: read it again
-                                const int e = c0 + 64 * r + lane;
-                                const int b = find_bin(L.pre, e);
-                                const int src = L.start[b] + e - (b ? L.pre[b - 1] : 0);
+                                int src, bu, off;
+                                candidate(64 * r + lane, src, bu, off);
                                 int u0, u1, u2, v0, v1, v2;
-                                dc_unpack(L.bu[b], u0, u1, u2);
+                                dc_unpack(bu, u0, u1, u2);
                                 dc_unpack(atoms[src].w, v0, v1, v2);
                                 t0 = u0 - v0;
                                 t1 = u1 - v1;
@@ -545,6 +646,7 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
                     }
                     if (lane == a) hcnt_lane = cnt;
                 }
+                if (CULL) wave_sync();
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -1412,8 +1514,15 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
                             nl->atoms_sorted.as<SortedAtom>(), nl->pos32.as<float4>(), nl->cell_start.as<int>(),
                             nl->scnt.as<int>(), nl->stage.as<int2>(), S, flags + 3, part);
         } else {
-            auto kern = ortho ? (B > 1 ? k_bin_pairs<true, true> : k_bin_pairs<true, false>)
-                              : (B > 1 ? k_bin_pairs<false, true> : k_bin_pairs<false, false>);
+            // Leaving out candidates costs a look at each: it pays for many
+            // home atoms (216 000 ions, 27 per wavefront: 407 -> 348 us) and
+            // for the small box of a few (1200 ions, one or two: 59 -> 50 us),
+            // not between (Cu, 15 per wavefront: 191 -> 198 us).
+            const double share = homes / nsub;
+            const bool cull = B == 1 && (share >= 20.0 || share <= 4.0);
+            auto kern = cull ? (ortho ? k_bin_pairs<true, false, true> : k_bin_pairs<false, false, true>)
+                             : ortho ? (B > 1 ? k_bin_pairs<true, true, false> : k_bin_pairs<true, false, false>)
+                                     : (B > 1 ? k_bin_pairs<false, true, false> : k_bin_pairs<false, false, false>);
             AGPU_LAUNCH("nl_pairs", kern, dim3(nbin_blk), dim3(TB), 0, s, B, nsub, g, C, cutoff_sq,
                         nl->atoms_sorted.as<SortedAtom>(), nl->cell_start.as<int>(), nl->scnt.as<int>(),
                         nl->stage.as<int2>(), S, flags + 3, part);
