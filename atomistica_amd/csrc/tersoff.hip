@@ -1124,8 +1124,9 @@ k_bop_rows_gather(int nat, const int *__restrict__ order, NlRows L, const double
 //                        written per record
 //   k_scr_slots          per entry of i's row: the total force i's terms put
 //                        on that neighbour (bond slot + records naming it)
+//                        and where a's row finds it (the reverse entry)
 //   k_scr_gather         f_a = own + sum over a's row of the slot the
-//                        neighbour wrote for a (through the reverse entry)
+//                        neighbour wrote for a
 // No atomics: every sum has one owner and a fixed order.
 // -------------------------------------------------------------------------
 // per element pair: the symmetric pair index (6 used), or the ordered one
@@ -1135,6 +1136,7 @@ struct ScrDev {
     double fin[9], fout[9], fbo[9];            // 1 / (r2 - r1) of the three cutoffs
     double Cmin[9], Cmax[9], dC[9], C_dr_cut[9], max_cut_sq[9];
     double ec, ed, efac2, eoff;                // exp_cutoff constants
+    double near_sq;                            // C_dr_cut r2^2 of the widest pair
 };
 
 constexpr int SCR_ROW = 256;       // row entries staged per atom
@@ -1168,13 +1170,21 @@ struct ScrShared {
 // One wavefront per atom, lanes over the row's entries; the row's vectors
 // r_j - r_i - A.n are staged in LDS.  FILL = false: keep flag and record
 // count; FILL = true: cutoffs and records at roff.
+//
+// The third atoms near i (|r_ik|^2 below near_sq, a handful) are walked first.
+// A bond inside its inner cutoff has all its third atoms among them, so that
+// walk is its reference walk; a longer bond that they already screen is
+// dropped whatever the rest would add (the terms of sij are negative, and a
+// dropped entry keeps nothing).  Only bonds that stay open walk the whole row,
+// from the start and in its order.  64 000 Si atoms, 46 entries a row:
+// 466 -> 118 us.
 template <bool FILL>
 __global__ void __launch_bounds__(256)
 k_scr_screen(ScrDev S, int nat_tot, const double *__restrict__ r, const int *__restrict__ el, int nel, int ordered,
              CellArg C,
              const int *__restrict__ offsets, const int2 *__restrict__ nbr, int *__restrict__ keep,
              int *__restrict__ rcnt, const int *__restrict__ roff, double4 *__restrict__ fcv,
-             int *__restrict__ rkn, double4 *__restrict__ rco, int *__restrict__ flags)
+             int *__restrict__ rkn, double4 *__restrict__ rco, int *__restrict__ from, int *__restrict__ flags)
 {
     __shared__ ScrShared sh[SCR_WAVES];
     ScrShared &L = sh[threadIdx.x >> 6];
@@ -1203,6 +1213,10 @@ k_scr_screen(ScrDev S, int nat_tot, const double *__restrict__ r, const int *__r
         L.e[t] = e;
     }
     __builtin_amdgcn_wave_barrier();
+    unsigned long long near_k[SCR_ROW / 64];
+#pragma unroll
+    for (int c = 0; c < SCR_ROW / 64; ++c)
+        near_k[c] = __ballot(64 * c + lane < n && L.r2[min(64 * c + lane, n - 1)] < S.near_sq);
     const double thr = -13.815510557964274;        // log(1e-6)
     const double dot_thr = 1e-10;
     for (int t = lane; t < n; t += 64) {
@@ -1229,17 +1243,19 @@ k_scr_screen(ScrDev S, int nat_tot, const double *__restrict__ r, const int *__r
                 double sij = 0.0, dsijdrij = 0.0;
                 const double Cmin = S.Cmin[typ], Cmax = S.Cmax[typ], dC = S.dC[typ];
                 const double lim = S.C_dr_cut[typ] * rl;
-                for (int u = 0; !(screened || sij < thr) && u < n; ++u) {
+                // one third atom; nothing when the bond is decided
+                auto third = [&](int u, bool record) {
+                    if (screened || sij < thr) return;
                     const double rlik = L.r2[u];
-                    if (!(rlik < lim)) continue;
+                    if (!(rlik < lim)) return;
                     const double rik[3] = {L.x[u], L.y[u], L.z[u]};
                     const int2 ek = L.e[u];
-                    if (ek.x == ej.x && ek.y == ej.y) continue;
+                    if (ek.x == ej.x && ek.y == ej.y) return;
                     const double dot_ij_ik = rij[0] * rik[0] + rij[1] * rik[1] + rij[2] * rik[2];
                     const double rjk[3] = {-rij[0] + rik[0], -rij[1] + rik[1], -rij[2] + rik[2]};
                     const double dot_ij_jk = rij[0] * rjk[0] + rij[1] * rjk[1] + rij[2] * rjk[2];
                     const double rljk = rjk[0] * rjk[0] + rjk[1] * rjk[1] + rjk[2] * rjk[2];
-                    if (!(dot_ij_ik > dot_thr && dot_ij_jk < -dot_thr)) continue;
+                    if (!(dot_ij_ik > dot_thr && dot_ij_jk < -dot_thr)) return;
                     const double xik = rlik / rl, xjk = rljk / rl;
                     const double xm = xik - xjk, xp = xik + xjk;
                     double fac = 1.0 / (1 - xm * xm);
@@ -1254,12 +1270,22 @@ k_scr_screen(ScrDev S, int nat_tot, const double *__restrict__ r, const int *__r
                         const double dCdrjk = 4 * xjk * fac * (1 - (Cv - 1) * xm);
                         fac = 2 * Cmax_C * dC / (C_Cmin * C_Cmin * C_Cmin);
                         dsijdrij = dsijdrij + fac * -(dCdrik + dCdrjk);
-                        if (FILL && cnt < qcap) {
+                        if (FILL && record && cnt < qcap) {
                             rkn[q0 + cnt] = beg + u;
                             rco[q0 + cnt] = make_double4(fac * dCdrik / rlik, fac * dCdrjk / rljk, 0.0, 0.0);
                         }
                         ++cnt;
                     }
+                };
+                const bool inner = lim <= S.near_sq;
+#pragma unroll
+                for (int c = 0; c < SCR_ROW / 64; ++c)
+                    for (unsigned long long m = near_k[c]; m; m &= m - 1) third(64 * c + __ffsll((long long)m) - 1, inner);
+                if (!inner && !(screened || sij < thr)) {
+                    need = false;
+                    sij = dsijdrij = 0.0;
+                    cnt = 0;
+                    for (int u = 0; !(screened || sij < thr) && u < n; ++u) third(u, true);
                 }
                 if ((screened || sij < thr) && rl > cin_h * cin_h) {
                     cnt = 0;              // fully screened: dropped
@@ -1309,6 +1335,7 @@ k_scr_screen(ScrDev S, int nat_tot, const double *__restrict__ r, const int *__r
             }
         }
         if (!FILL) {
+            if (from) from[s] = -1;
             if (kept) fcv[s] = make_double4(fcar, dfcar, fcbo, dfcbo);
             keep[s] = kept;
             rcnt[s] = kept ? cnt : 0;
@@ -1623,33 +1650,69 @@ k_bop_scr(TersoffDev P, ScrDev S, int nat, const int *__restrict__ order, const 
 
 // wavefront per atom, lanes over its row: total force the atom's terms put
 // on each neighbour entry (bond slot + records naming the entry, in record
-// order)
+// order).  With from, an entry i->j that carries any is entered at its reverse
+// entry j->i (the wavefront looks through j's row together), and the others
+// are left out: about 4 of 46 entries in a crystal, where the reverse of every
+// entry, looked up beforehand, took 232 us on 64 000 atoms (this pass: 54 us).
 __global__ void __launch_bounds__(256)
-k_scr_slots(int nat, const int *__restrict__ offsets, const int *__restrict__ keep,
+k_scr_slots(int nat, const int *__restrict__ offsets, const int2 *__restrict__ nbr, const int *__restrict__ keep,
             const double *__restrict__ fslot, const int *__restrict__ roff, const int *__restrict__ rkn,
-            const double *__restrict__ frec, double *__restrict__ fsl)
+            const double *__restrict__ frec, double *__restrict__ fsl, int *__restrict__ from,
+            int *__restrict__ flags)
 {
     const int lane = threadIdx.x & 63;
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= nat) return;
     const int beg = offsets[i], end = offsets[i + 1];
     const int q0 = roff[beg], q1 = roff[end];
-    for (int s = beg + lane; s < end; s += 64) {
+    for (int base = beg; base < end; base += 64) {
+        const int s = base + lane;
         double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-        if (keep[s]) {
-            a0 = fslot[3 * (size_t)s];
-            a1 = fslot[3 * (size_t)s + 1];
-            a2 = fslot[3 * (size_t)s + 2];
-        }
-        for (int q = q0; q < q1; ++q)
-            if (rkn[q] == s) {
-                a0 += frec[3 * (size_t)q];
-                a1 += frec[3 * (size_t)q + 1];
-                a2 += frec[3 * (size_t)q + 2];
+        bool any = false;
+        if (s < end) {
+            if (keep[s]) {
+                any = true;
+                a0 = fslot[3 * (size_t)s];
+                a1 = fslot[3 * (size_t)s + 1];
+                a2 = fslot[3 * (size_t)s + 2];
             }
-        fsl[3 * (size_t)s] = a0;
-        fsl[3 * (size_t)s + 1] = a1;
-        fsl[3 * (size_t)s + 2] = a2;
+            for (int q = q0; q < q1; ++q)
+                if (rkn[q] == s) {
+                    any = true;
+                    a0 += frec[3 * (size_t)q];
+                    a1 += frec[3 * (size_t)q + 1];
+                    a2 += frec[3 * (size_t)q + 2];
+                }
+            if (any || !from) {
+                fsl[3 * (size_t)s] = a0;
+                fsl[3 * (size_t)s + 1] = a1;
+                fsl[3 * (size_t)s + 2] = a2;
+            }
+        }
+        if (!from) continue;
+        const int2 e = s < end ? nbr[s] : make_int2(0, 0);
+        int o0 = 0, o1 = 0;
+        if (any) {
+            o0 = offsets[e.x];
+            o1 = offsets[e.x + 1];
+        }
+        for (unsigned long long m = __ballot(any); m; m &= m - 1) {
+            const int u = __ffsll((long long)m) - 1;
+            int a, b, c;
+            dc_unpack(__builtin_amdgcn_readlane(e.y, u), a, b, c);
+            const int want = dc_pack(-a, -b, -c);
+            const int r1 = __builtin_amdgcn_readlane(o1, u);
+            bool found = false;
+            for (int r0 = __builtin_amdgcn_readlane(o0, u); r0 < r1 && !found; r0 += 64) {
+                const int2 f = r0 + lane < r1 ? nbr[r0 + lane] : make_int2(-1, 0);
+                const unsigned long long hit = __ballot(f.x == i && f.y == want);
+                if (hit) {
+                    found = true;
+                    if (lane == 0) from[r0 + __ffsll((long long)hit) - 1] = base + u;
+                }
+            }
+            if (!found && lane == 0) atomicOr(flags, DERR_BOND_OVERFLOW);
+        }
     }
 }
 
@@ -1891,6 +1954,7 @@ static void derive_scr(ScrDev &S, const TersoffDev &D, const agpu_screening_para
         S.C_dr_cut[q] = sp.Cmax[q] > 2.0 ? sp.Cmax[q] * sp.Cmax[q] / (4 * (sp.Cmax[q] - 1)) : 1.0;
         double mx = std::max(S.r2[q], std::max(S.or2[q], S.bor2[q]));
         S.max_cut_sq[q] = mx * mx;
+        S.near_sq = std::max(S.near_sq, S.C_dr_cut[q] * (S.r2[q] * S.r2[q]));
     }
     // exp_cutoff_init (cutoff.f90:245-258)
     const double v1 = std::exp(-8.0), dv1 = -24 * v1, ddv1 = -48 * v1 - 24 * dv1;
@@ -1989,13 +2053,17 @@ static int tersoff_scr_compute(agpu_potential *pot, const agpu_eval_args *a)
     const int *offs = nl->offsets.as<int>();
     const int2 *nbr = nl->nbr.as<int2>();
     const dim3 gw((unsigned)((nat + SCR_WAVES - 1) / SCR_WAVES));
+    // The entries that carry a force are entered at their reverse entries by
+    // k_scr_slots; an imported list, whose rows need not come in pairs, has
+    // every reverse entry looked up and checked first.
+    const bool push = !nl->external;
     // pass 1: keep flags, cutoffs and record counts; exclusive scan to record
     // offsets
     AGPU_CHECK(zero_dev(st->rcnt.as<int>() + E, sizeof(int)));
     AGPU_LAUNCH("scr_count", k_scr_screen<false>, gw, dim3(256), 0, s, S, nat, p->d_r, el, st->prm.nel,
                 (int)(st->dev.fam == 3), C, offs,
                 nbr, st->keep.as<int>(), st->rcnt.as<int>(), nullptr, st->fcv.as<double4>(), nullptr, nullptr,
-                dstats);
+                push ? st->nlrev.as<int>() : nullptr, dstats);
     size_t tmp = 0;
     AGPU_HIP(rocprim::exclusive_scan(nullptr, tmp, st->rcnt.as<int>(), st->roff.as<int>(), 0, (size_t)E + 1,
                                      rocprim::plus<int>(), s));
@@ -2015,11 +2083,13 @@ static int tersoff_scr_compute(agpu_potential *pot, const agpu_eval_args *a)
     AGPU_LAUNCH("scr_fill", k_scr_screen<true>, gw, dim3(256), 0, s, S, nat, p->d_r, el, st->prm.nel,
                 (int)(st->dev.fam == 3), C, offs, nbr,
                 st->keep.as<int>(), st->rcnt.as<int>(), st->roff.as<int>(), st->fcv.as<double4>(),
-                st->rkn.as<int>(), st->rco.as<double4>(), dstats);
+                st->rkn.as<int>(), st->rco.as<double4>(), nullptr, dstats);
     AGPU_LAUNCH("scr_bonds", k_scr_bonds, dim3((nat + 255) / 256), dim3(256), 0, s, nat, offs, st->keep.as<int>(),
                 st->bslot.as<int>(), st->bcnt.as<int>());
     // reverse entries of the list, once per list build
-    if (st->nlrev_nl != nl || st->nlrev_upd != nl->n_updates) {
+    if (push) {
+        st->nlrev_nl = nullptr;
+    } else if (st->nlrev_nl != nl || st->nlrev_upd != nl->n_updates) {
         AGPU_LAUNCH("scr_rev", k_nl_rev_entries, gw, dim3(256), 0, s, nat, offs, nbr, st->nlrev.as<int>(), dstats);
         st->nlrev_nl = nl;
         st->nlrev_upd = nl->n_updates;
@@ -2042,14 +2112,17 @@ static int tersoff_scr_compute(agpu_potential *pot, const agpu_eval_args *a)
         AGPU_CHECK(dispatch_bop_scr<float>(G, st, S, nat, order, p->d_r, el, C, nl, a->mask, a, s, &nblk));
     else
         AGPU_CHECK(dispatch_bop_scr<double>(G, st, S, nat, order, p->d_r, el, C, nl, a->mask, a, s, &nblk));
-    AGPU_LAUNCH("scr_slots", k_scr_slots, gw, dim3(256), 0, s, nat, offs, st->keep.as<int>(),
+    AGPU_LAUNCH("scr_slots", k_scr_slots, gw, dim3(256), 0, s, nat, offs, nbr, st->keep.as<int>(),
                 st->fslot.as<double>(), st->roff.as<int>(), st->rkn.as<int>(), st->frec.as<double>(),
-                st->fsl.as<double>());
+                st->fsl.as<double>(), push ? st->nlrev.as<int>() : nullptr, dstats);
     AGPU_LAUNCH("scr_gather", k_scr_gather, dim3((unsigned)((nat + 256 / SCR_GL - 1) / (256 / SCR_GL))), dim3(256), 0,
                 s, nat, offs, st->nlrev.as<int>(), st->keep.as<int>(), st->fsl.as<double>(), st->fown.as<double>(),
                 st->eslot.as<double>(), st->wslot.as<double>(), a->f, a->epot_per_at, a->wpot_per_at);
     AGPU_CHECK(reduce_ev(st->partial.as<double>(), nblk, 10, a->epot, a->wpot, nullptr));
+    AGPU_HIP(hipMemcpyAsync(pot->stats.h + 1, dstats, sizeof(int), hipMemcpyDeviceToHost, s));
     AGPU_HIP(hipStreamSynchronize(s));
+    if (pot->stats.h[1] & DERR_BOND_OVERFLOW)
+        return set_error(AGPU_ERR_NEB, "screened bond order: list entry without its reverse entry");
     return AGPU_OK;
 }
 

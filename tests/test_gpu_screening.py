@@ -114,3 +114,32 @@ def test_screened_mixed_error():
     rms = float(np.sqrt(np.mean((f32 - f64) ** 2)))
     print("screened mixed: F rms %.3e  |dE|/N %.3e" % (rms, abs(e32 - e64) / len(pos)), flush=True)
     assert rms <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+@pytest.mark.parametrize("seed", range(3))
+def test_near_third_atoms_first(n, seed):
+    """Bonds decided by the near third atoms, inside and outside the inner
+    cut-off, and bonds that walk the whole row: dense random Si from one to
+    some hundred atoms, rows below, at and above 64 and 128 entries."""
+    from atomistica_amd import native as N
+    from atomistica_amd import parameters as P
+    from oracle import oracle as O
+    rng = np.random.default_rng(10 * n + seed)
+    cell = np.diag([4.2 * n, 4.4 * n, 4.6 * n]) + 0.1 * n * rng.uniform(-1, 1, (3, 3))
+    m = [6, 9, 14][seed] * n ** 3 // 2 + 1
+    pos = rng.random((m, 3)) @ cell
+    print("near third atoms", n, seed, m, flush=True)
+    rc = 6.0 * np.sqrt(9.0 / 8.0)
+    onl = O.nl_build(pos, cell, [True] * 3, rc, avgn=600)
+    if np.diff(onl[0]).max() > 256:
+        pytest.skip("rows beyond 256 entries are refused")
+    e0, f0, w0 = O.tersoff(P.Tersoff_PRB_39_5566_Si_C__Scr, pos, np.ones(m, np.int32), cell, onl)[:3]
+    p = N.from_atoms(pos, cell, [True] * 3, np.full(m, 14, np.int32))
+    nl = N.Neighbors(600)
+    pot = N.TersoffScr()
+    pot.bind_to(p, nl)
+    e, f, w = pot.energy_and_forces(p, nl)[:3]
+    assert abs(e - e0) <= 1e-10 * max(1.0, abs(e0))
+    assert np.abs(f - f0).max() <= 1e-10 * max(1.0, np.abs(f0).max())
+    assert np.abs(w - w0).max() <= 1e-10 * max(1.0, np.abs(w0).max())
