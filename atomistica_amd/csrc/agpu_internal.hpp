@@ -61,6 +61,20 @@ struct DevBuf {
     ~DevBuf() { release(); }
 };
 
+// Grow-only pinned host buffer owned by a handle, for copies that the host
+// does not wait for: wait() before it is written again.
+struct HostBuf {
+    void *ptr = nullptr;
+    size_t bytes = 0;
+    hipEvent_t done = nullptr;
+    bool busy = false;
+    int reserve(size_t nbytes);
+    int mark(hipStream_t s);      // the copy just queued on s reads or fills it
+    int wait();
+    template <typename T> T *as() const { return static_cast<T *>(ptr); }
+    ~HostBuf();
+};
+
 // Pinned host staging word for flags and small statistics.
 struct HostStats {
     int *h = nullptr;
@@ -318,6 +332,9 @@ struct agpu_potential {
     void (*free_impl)(void *) = nullptr;
     agpu::DevBuf d_el, flags, partial, partial_out;
     agpu::HostStats stats;
+    // one block for the arrays of a call with host arrays
+    agpu::DevBuf io;
+    agpu::HostBuf h_io;
 };
 
 namespace agpu {

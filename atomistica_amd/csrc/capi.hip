@@ -67,6 +67,40 @@ void DevBuf::release()
     bytes = 0;
 }
 
+int HostBuf::reserve(size_t nbytes)
+{
+    if (nbytes <= bytes && ptr) return AGPU_OK;
+    AGPU_CHECK(wait());
+    if (ptr) (void)hipHostFree(ptr);
+    ptr = nullptr;
+    bytes = 0;
+    AGPU_HIP(hipHostMalloc(&ptr, nbytes, hipHostMallocDefault));
+    bytes = nbytes;
+    return AGPU_OK;
+}
+
+int HostBuf::mark(hipStream_t s)
+{
+    if (!done) AGPU_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    AGPU_HIP(hipEventRecord(done, s));
+    busy = true;
+    return AGPU_OK;
+}
+
+int HostBuf::wait()
+{
+    if (busy) AGPU_HIP(hipEventSynchronize(done));
+    busy = false;
+    return AGPU_OK;
+}
+
+HostBuf::~HostBuf()
+{
+    (void)wait();
+    if (done) (void)hipEventDestroy(done);
+    if (ptr) (void)hipHostFree(ptr);
+}
+
 int HostStats::init()
 {
     if (h) return AGPU_OK;
@@ -92,6 +126,11 @@ struct ProfRec {
 static bool g_prof = false;
 static std::vector<ProfRec> g_prof_recs;
 static std::map<std::string, std::pair<double, int>> g_prof_done;
+
+// Host arrays of a call up to this size go through one pinned block: one copy
+// each way instead of one per array.  Larger ones are copied from where they
+// are, so that the pinned block stays small.
+constexpr size_t IO_PACKED = 4u << 20;
 
 // while a step is being captured into a graph: no host synchronisation, no
 // memset nodes, no profiling events (set by the MD driver)
@@ -691,54 +730,71 @@ static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors
         AGPU_CHECK(nl_update(nl, p, 0));
         nbond = nl->total;
     }
-    DevBuf st;
-    size_t n = 1 + 3 * (size_t)nat + 9 + (a.q ? nat : 0) + (a.epot_per_at ? nat : 0) +
-               (a.wpot_per_at ? 9 * (size_t)nat : 0) + (a.epot_per_bond ? (size_t)nbond : 0) +
-               (a.f_per_bond ? 3 * (size_t)nbond : 0) + (a.wpot_per_bond ? 9 * (size_t)nbond : 0);
-    size_t nmask = a.mask ? (size_t)nat : 0;
-    AGPU_CHECK(st.reserve(sizeof(double) * n + sizeof(int) * (nmask + 1)));
-    double *b = st.as<double>();
+    const size_t n = 1 + 3 * (size_t)nat + 9 + (a.q ? nat : 0) + (a.epot_per_at ? nat : 0) +
+                     (a.wpot_per_at ? 9 * (size_t)nat : 0) + (a.epot_per_bond ? (size_t)nbond : 0) +
+                     (a.f_per_bond ? 3 * (size_t)nbond : 0) + (a.wpot_per_bond ? 9 * (size_t)nbond : 0);
+    const size_t nmask = a.mask ? (size_t)nat : 0, size = sizeof(double) * n + sizeof(int) * nmask;
+    AGPU_CHECK(pot->io.reserve(size + sizeof(int)));
+    const bool packed = size <= IO_PACKED;
+    double *const base = pot->io.as<double>();
+    // the block: what comes back (host array, length), then q and the mask
+    struct Part {
+        double *host, *dev;
+        size_t len;
+    } part[8];
+    int np = 0;
+    double *cur = base;
+    auto take = [&](double *h, size_t len, bool used) -> double * {
+        if (!used) return nullptr;
+        part[np++] = Part{h, cur, len};
+        cur += len;
+        return part[np - 1].dev;
+    };
     agpu_eval_args d = a;
     d.flags &= ~AGPU_HOST;
-    double *cur = b;
-    d.epot = cur;
-    cur += 1;
-    d.f = cur;
-    cur += 3 * (size_t)nat;
-    d.wpot = cur;
-    cur += 9;
-    double *qd = nullptr, *epa = nullptr, *wpa = nullptr;
-    if (a.q) { qd = cur; cur += nat; }
-    if (a.epot_per_at) { epa = cur; cur += nat; }
-    if (a.wpot_per_at) { wpa = cur; cur += 9 * (size_t)nat; }
-    double *epb = nullptr, *fpb = nullptr, *wpb = nullptr;
-    if (a.epot_per_bond) { epb = cur; cur += nbond; }
-    if (a.f_per_bond) { fpb = cur; cur += 3 * (size_t)nbond; }
-    if (a.wpot_per_bond) { wpb = cur; cur += 9 * (size_t)nbond; }
-    d.epot_per_bond = epb;
-    d.f_per_bond = fpb;
-    d.wpot_per_bond = wpb;
-    int *md = a.mask ? reinterpret_cast<int *>(cur) : nullptr;
+    d.epot = take(a.epot, 1, true);
+    d.f = take(a.f, 3 * (size_t)nat, true);
+    d.wpot = take(a.wpot, 9, true);
+    d.epot_per_at = take(a.epot_per_at, nat, a.epot_per_at);
+    d.wpot_per_at = take(a.wpot_per_at, 9 * (size_t)nat, a.wpot_per_at);
+    d.epot_per_bond = take(a.epot_per_bond, nbond, a.epot_per_bond);
+    d.f_per_bond = take(a.f_per_bond, 3 * (size_t)nbond, a.f_per_bond);
+    d.wpot_per_bond = take(a.wpot_per_bond, 9 * (size_t)nbond, a.wpot_per_bond);
+    const size_t back = (size_t)(cur - base);
+    double *qd = nullptr;
+    if (a.q) {
+        qd = cur;
+        cur += nat;
+    }
     d.q = qd;
-    d.epot_per_at = epa;
-    d.wpot_per_at = wpa;
+    int *md = a.mask ? reinterpret_cast<int *>(cur) : nullptr;
     d.mask = md;
     hipStream_t s = stream();
-    AGPU_HIP(hipMemsetAsync(d.epot, 0, sizeof(double), s));
-    if (a.f) AGPU_HIP(hipMemcpyAsync(d.f, a.f, sizeof(double) * 3 * nat, hipMemcpyHostToDevice, s));
-    else AGPU_HIP(hipMemsetAsync(d.f, 0, sizeof(double) * 3 * nat, s));
-    if (a.wpot) AGPU_HIP(hipMemcpyAsync(d.wpot, a.wpot, sizeof(double) * 9, hipMemcpyHostToDevice, s));
-    else AGPU_HIP(hipMemsetAsync(d.wpot, 0, sizeof(double) * 9, s));
-    if (a.q) AGPU_HIP(hipMemcpyAsync(qd, a.q, sizeof(double) * nat, hipMemcpyHostToDevice, s));
-    if (epa) AGPU_HIP(hipMemcpyAsync(epa, a.epot_per_at, sizeof(double) * nat, hipMemcpyHostToDevice, s));
-    if (wpa) AGPU_HIP(hipMemcpyAsync(wpa, a.wpot_per_at, sizeof(double) * 9 * nat, hipMemcpyHostToDevice, s));
-    if (md) AGPU_HIP(hipMemcpyAsync(md, a.mask, sizeof(int) * nat, hipMemcpyHostToDevice, s));
-    if (epb && nbond)
-        AGPU_HIP(hipMemcpyAsync(epb, a.epot_per_bond, sizeof(double) * nbond, hipMemcpyHostToDevice, s));
-    if (fpb && nbond)
-        AGPU_HIP(hipMemcpyAsync(fpb, a.f_per_bond, sizeof(double) * 3 * nbond, hipMemcpyHostToDevice, s));
-    if (wpb && nbond)
-        AGPU_HIP(hipMemcpyAsync(wpb, a.wpot_per_bond, sizeof(double) * 9 * nbond, hipMemcpyHostToDevice, s));
+    if (packed) {
+        AGPU_CHECK(pot->h_io.wait());
+        AGPU_CHECK(pot->h_io.reserve(size));
+        double *h = pot->h_io.as<double>();
+        for (int k = 0; k < np; ++k) {
+            double *o = h + (part[k].dev - base);
+            // epot is set; the other arrays are added to
+            if (k > 0 && part[k].host) std::memcpy(o, part[k].host, sizeof(double) * part[k].len);
+            else std::memset(o, 0, sizeof(double) * part[k].len);
+        }
+        if (a.q) std::memcpy(h + (qd - base), a.q, sizeof(double) * nat);
+        if (md) std::memcpy(h + (reinterpret_cast<double *>(md) - base), a.mask, sizeof(int) * nat);
+        AGPU_HIP(hipMemcpyAsync(base, h, size, hipMemcpyHostToDevice, s));
+        AGPU_CHECK(pot->h_io.mark(s));
+    } else {
+        for (int k = 0; k < np; ++k) {
+            if (!part[k].len) continue;
+            if (k > 0 && part[k].host)
+                AGPU_HIP(hipMemcpyAsync(part[k].dev, part[k].host, sizeof(double) * part[k].len, hipMemcpyHostToDevice, s));
+            else
+                AGPU_HIP(hipMemsetAsync(part[k].dev, 0, sizeof(double) * part[k].len, s));
+        }
+        if (a.q) AGPU_HIP(hipMemcpyAsync(qd, a.q, sizeof(double) * nat, hipMemcpyHostToDevice, s));
+        if (md) AGPU_HIP(hipMemcpyAsync(md, a.mask, sizeof(int) * nat, hipMemcpyHostToDevice, s));
+    }
     switch (pot->kind) {
     case AGPU_KIND_TERSOFF:
     case AGPU_KIND_KUMAGAI:
@@ -756,19 +812,20 @@ static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors
     default: rc = set_error(AGPU_ERR_STATE, "unknown potential kind");
     }
     if (rc != AGPU_OK) return rc;
-    if (a.epot) AGPU_HIP(hipMemcpyAsync(a.epot, d.epot, sizeof(double), hipMemcpyDeviceToHost, s));
-    if (a.f) AGPU_HIP(hipMemcpyAsync(a.f, d.f, sizeof(double) * 3 * nat, hipMemcpyDeviceToHost, s));
-    if (a.wpot) AGPU_HIP(hipMemcpyAsync(a.wpot, d.wpot, sizeof(double) * 9, hipMemcpyDeviceToHost, s));
-    if (epa) AGPU_HIP(hipMemcpyAsync(a.epot_per_at, epa, sizeof(double) * nat, hipMemcpyDeviceToHost, s));
-    if (wpa) AGPU_HIP(hipMemcpyAsync(a.wpot_per_at, wpa, sizeof(double) * 9 * nat, hipMemcpyDeviceToHost, s));
-    if (nl->total != nbond && (epb || fpb || wpb))
+    if (nl->total != nbond && (a.epot_per_bond || a.f_per_bond || a.wpot_per_bond))
         return set_error(AGPU_ERR_STATE, "energy_and_forces: the list changed size during the call");
-    if (epb && nbond)
-        AGPU_HIP(hipMemcpyAsync(a.epot_per_bond, epb, sizeof(double) * nbond, hipMemcpyDeviceToHost, s));
-    if (fpb && nbond)
-        AGPU_HIP(hipMemcpyAsync(a.f_per_bond, fpb, sizeof(double) * 3 * nbond, hipMemcpyDeviceToHost, s));
-    if (wpb && nbond)
-        AGPU_HIP(hipMemcpyAsync(a.wpot_per_bond, wpb, sizeof(double) * 9 * nbond, hipMemcpyDeviceToHost, s));
+    if (packed) {
+        double *h = pot->h_io.as<double>();
+        AGPU_CHECK(pot->h_io.wait());
+        AGPU_HIP(hipMemcpyAsync(h, base, sizeof(double) * back, hipMemcpyDeviceToHost, s));
+        AGPU_HIP(hipStreamSynchronize(s));
+        for (int k = 0; k < np; ++k)
+            if (part[k].host) std::memcpy(part[k].host, h + (part[k].dev - base), sizeof(double) * part[k].len);
+        return AGPU_OK;
+    }
+    for (int k = 0; k < np; ++k)
+        if (part[k].host && part[k].len)
+            AGPU_HIP(hipMemcpyAsync(part[k].host, part[k].dev, sizeof(double) * part[k].len, hipMemcpyDeviceToHost, s));
     AGPU_HIP(hipStreamSynchronize(s));
     return AGPU_OK;
 }
