@@ -12,7 +12,7 @@ struct agpu_batch {
     int ntot = 0;
     std::vector<int> h_off;        // atom offsets (nstruct + 1)
     std::vector<double> h_cell;    // 9 per structure: cell[9*s + 3*k + x]
-    agpu::DevBuf off, sof, cell, rec, r, counts, offsets, nbr, scan_tmp, eatom,
+    agpu::DevBuf off, sof, cell, rec, r, u, counts, offsets, nbr, scan_tmp, eatom,
         partial, gacc, flags;
     // per list entry: bond i -> j as {unit vector, length} in FP64 and FP32,
     // the index of the reverse entry j -> i (-1 if absent) and the owner i
@@ -39,3 +39,36 @@ struct agpu_batch {
         if (ewb && ewb_free) ewb_free(ewb);
     }
 };
+
+namespace agpu {
+// Fractional coordinates per atom into b->u, in units of 2^-32 of a lattice
+// vector: the difference of two, taken modulo 2^32 as a signed number, is the
+// difference to the nearest image along each axis.
+int batch_fractions(agpu_batch *b);
+
+// the wrapped difference of two of them as fractions of the lattice vectors
+__device__ __forceinline__ void batch_diff(const int4 &a, const int4 &b, int (&d)[3])
+{
+    d[0] = (int)((unsigned)a.x - (unsigned)b.x);
+    d[1] = (int)((unsigned)a.y - (unsigned)b.y);
+    d[2] = (int)((unsigned)a.z - (unsigned)b.z);
+}
+
+constexpr double BATCH_TURN = 2.3283064365386963e-10;    // 2^-32
+
+// Images around the nearest one that come within rc of an atom of a cell with
+// reciprocal vectors b (m per axis), and the screening radius in FP32: a
+// difference vector formed there is off by a few 2^-24 of its summands.
+__device__ __forceinline__ float batch_reach(const double *A, const double *b, double rc, int (&m)[3])
+{
+    float reach = 0.f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double t = rc * sqrt(b[3 * k] * b[3 * k] + b[3 * k + 1] * b[3 * k + 1] + b[3 * k + 2] * b[3 * k + 2]);
+        m[k] = max(0, (int)ceil(t - 0.5 + 1e-6));
+        const float len = (float)sqrt(A[3 * k] * A[3 * k] + A[3 * k + 1] * A[3 * k + 1] + A[3 * k + 2] * A[3 * k + 2]);
+        reach += (0.5f + m[k]) * len;
+    }
+    return (float)rc * 1.000001f + 1e-6f * reach;
+}
+}  // namespace agpu

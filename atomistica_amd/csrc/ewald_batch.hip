@@ -31,7 +31,7 @@ struct EwbState {
     double kmax = 0.0;
     uint64_t struct_rev = ~0ull;
     EwrState recip;
-    DevBuf d_u, d_ionrec, d_krec, d_q;
+    DevBuf d_ionrec, d_krec, d_q;
 };
 
 static void ewb_free(void *p) { delete static_cast<EwbState *>(p); }
@@ -44,26 +44,6 @@ struct EwbGeom {
     const double *cell;    // 9 per structure, cell[3k+x] = a_k[x]
     const double *rec;     // 9 per structure, rec[3k+x] = b_k[x], a_k . b_l = delta_kl
 };
-
-// Fractional coordinates per ion in units of 2^-32 of a lattice vector: the
-// difference of two, taken modulo 2^32 as a signed number, is the difference
-// to the nearest image along each axis.
-__global__ void k_ewb_frac(int n, const int *__restrict__ sof, const double *__restrict__ rec,
-                           const double *__restrict__ r, int4 *__restrict__ u)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const double *b = rec + 9 * (size_t)sof[j];
-    const double x = r[3 * (size_t)j], y = r[3 * (size_t)j + 1], z = r[3 * (size_t)j + 2];
-    int v[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        double s = b[3 * k] * x + b[3 * k + 1] * y + b[3 * k + 2] * z;
-        s -= floor(s);
-        v[k] = (int)(unsigned)(long long)(s * 4294967296.0);
-    }
-    u[j] = make_int4(v[0], v[1], v[2], 0);
-}
 
 // A wavefront per ion.  The lanes screen 64 ions of the structure at a time
 // in FP32 (with slack for the rounding), for the nearest image and, in cells
@@ -88,26 +68,15 @@ k_ewb_real(int n, const int *__restrict__ sof, EwbGeom G, const double *__restri
     int2 *Q = queue[wave];
     double A[9], b[9];
     int m[3];
-    float Af[9], reach = 0.f;
+    float Af[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
         A[k] = G.cell[9 * (size_t)st + k];
         b[k] = G.rec[9 * (size_t)st + k];
+        Af[k] = (float)A[k];
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const double t =
-            cutoff * sqrt(b[3 * k] * b[3 * k] + b[3 * k + 1] * b[3 * k + 1] + b[3 * k + 2] * b[3 * k + 2]);
-        // images around the nearest one that can come within the cut-off
-        m[k] = max(0, (int)ceil(t - 0.5 + 1e-6));
-        const float len = (float)sqrt(A[3 * k] * A[3 * k] + A[3 * k + 1] * A[3 * k + 1] + A[3 * k + 2] * A[3 * k + 2]);
-        reach += (0.5f + m[k]) * len;
-#pragma unroll
-        for (int x = 0; x < 3; ++x) Af[3 * k + x] = (float)(A[3 * k + x]);
-    }
+    const float rs = batch_reach(A, b, cutoff, m), rs2 = rs * rs;
     const double rc2 = cutoff * cutoff;
-    // FP32 rounding of a difference vector: a few 2^-24 of its summands
-    const float rs = (float)cutoff * 1.000001f + 1e-6f * reach, rs2 = rs * rs;
     const double sap = beta / sqrt(M_PI);
     const double ri[3] = {r[3 * (size_t)i], r[3 * (size_t)i + 1], r[3 * (size_t)i + 2]};
     const double qi = q[i];
@@ -124,14 +93,14 @@ k_ewb_real(int n, const int *__restrict__ sof, EwbGeom G, const double *__restri
         if (!(fabs(qj) > 1e-10)) return;
         const int4 uj = u[j];
         const double d0[3] = {ri[0] - r[3 * (size_t)j], ri[1] - r[3 * (size_t)j + 1], ri[2] - r[3 * (size_t)j + 2]};
-        const int du[3] = {(int)((unsigned)ui.x - (unsigned)uj.x), (int)((unsigned)ui.y - (unsigned)uj.y),
-                           (int)((unsigned)ui.z - (unsigned)uj.z)};
+        int du[3];
+        batch_diff(ui, uj, du);
         double nk[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             // the whole turns between the difference and its wrapped form
             const double ds = b[3 * k] * d0[0] + b[3 * k + 1] * d0[1] + b[3 * k + 2] * d0[2];
-            nk[k] = rint((double)du[k] * 2.3283064365386963e-10 - ds) + (double)(((c.y >> (10 * k)) & 1023) - 512);
+            nk[k] = rint((double)du[k] * BATCH_TURN - ds) + (double)(((c.y >> (10 * k)) & 1023) - 512);
         }
         if (j == i && nk[0] == 0.0 && nk[1] == 0.0 && nk[2] == 0.0) return;
         double d[3];
@@ -165,9 +134,10 @@ k_ewb_real(int n, const int *__restrict__ sof, EwbGeom G, const double *__restri
             for (int c = 0; c < EWB_C; ++c) uj[c] = u[min(base + 64 * c + lane, a1 - 1)];
 #pragma unroll
             for (int c = 0; c < EWB_C; ++c) {
-                du[c][0] = (float)(int)((unsigned)ui.x - (unsigned)uj[c].x) * 2.3283064e-10f;
-                du[c][1] = (float)(int)((unsigned)ui.y - (unsigned)uj[c].y) * 2.3283064e-10f;
-                du[c][2] = (float)(int)((unsigned)ui.z - (unsigned)uj[c].z) * 2.3283064e-10f;
+                int d[3];
+                batch_diff(ui, uj[c], d);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) du[c][k] = (float)d[k] * (float)BATCH_TURN;
             }
             for (int o = 0; o < ncomb; ++o) {
                 const int n0 = o / (w1 * w2) - m[0], n1 = (o / w2) % w1 - m[1], n2 = o % w2 - m[2];
@@ -307,10 +277,8 @@ extern "C" int agpu_ewald_batch_compute(agpu_batch *b, const double *q, double c
     AGPU_CHECK(st.d_krec.reserve(sizeof(double) * 10 * ((size_t)st.recip.ntile + 1)));
     EwbGeom G{b->off.as<int>(), b->cell.as<double>(), b->rec.as<double>()};
     if (n > 0) {
-        AGPU_CHECK(st.d_u.reserve(sizeof(int4) * (size_t)n));
-        int4 *u = st.d_u.as<int4>();
-        AGPU_LAUNCH("ewald_batch_frac", k_ewb_frac, dim3((n + 255) / 256), dim3(256), 0, s, n, b->sof.as<int>(),
-                    b->rec.as<double>(), b->r.as<double>(), u);
+        AGPU_CHECK(batch_fractions(b));
+        const int4 *u = b->u.as<int4>();
         const dim3 g((n + EWB_W - 1) / EWB_W), t(64 * EWB_W);
         if (precision == AGPU_PREC_MIXED)
             AGPU_LAUNCH("ewald_batch_real_mixed", k_ewb_real<float>, g, t, 0, s, n, b->sof.as<int>(), G,

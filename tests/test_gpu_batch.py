@@ -186,3 +186,33 @@ def test_batch_full_set_4096():
         a0, a1 = b.offsets[s], b.offsets[s + 1]
         assert np.abs(f64[a0:a1].sum(0)).max() < 1e-9
         assert np.abs(fn[a0:a1].sum(0)).max() < 1e-4
+
+
+def test_batch_list_edges():
+    """The wavefront-per-atom list: structures of one atom up to beyond two 64
+    atom trips, cells from a fraction of the cut-off (images on all sides, the
+    atom's own among them) to several of it, sheared, atoms many cells away."""
+    from oracle import oracle as O
+    from atomistica_amd import parameters as P
+    from atomistica_amd.batch import TersoffBatch, params_from_theta, theta_from_params
+    th = theta_from_params(P.Tersoff_Si)
+    prm = params_from_theta(th)
+    rng = np.random.default_rng(17)
+    S = []
+    for n, edge in ((1, 2.3), (1, 2.9), (2, 4.0), (3, 4.6), (63, 11.0), (64, 10.5), (65, 12.5), (130, 14.0), (200, 31.0)):
+        cell = np.diag([edge, 1.1 * edge, 0.95 * edge]) @ (np.eye(3) + rng.uniform(-0.2, 0.2, (3, 3)))
+        pos = W.random_positions(n, cell, 1.7, int(rng.integers(1 << 30)))
+        S.append((pos + rng.integers(-30, 31, (n, 3)) @ cell, cell))
+    b = TersoffBatch(S)
+    e, f = (t.cpu().numpy() for t in b.forward(th))
+    pairs = 0
+    for s, (pos, cell) in enumerate(S):
+        print("batch list", s, len(pos), flush=True)
+        # the list is built at 1.02 S
+        pairs += len(O.nl_build(pos, cell, [True] * 3, 1.02 * th[10], avgn=400)[1])
+        onl = O.nl_build(pos, cell, [True] * 3, th[10], avgn=400)
+        e0, f0 = O.tersoff(prm, pos, np.zeros(len(pos), np.int32), cell, onl)[:2]
+        a = slice(b.offsets[s], b.offsets[s + 1])
+        assert abs(e[s] - e0) <= 1e-10 * max(1.0, abs(e0)), s
+        assert np.abs(f[a] - f0).max() <= 1e-10 * max(1.0, np.abs(f0).max()), s
+    assert b.pairs() == pairs
