@@ -128,6 +128,7 @@ struct EamState {
     // lanes per atom and entries per lane of the single-element kernels
     // (chosen by eam_autotune; the defaults otherwise)
     int tg = 16, tu = 4;
+    int ncu = 256;                // CUs: workgroups of the passes with the table in LDS
 };
 
 static void eam_free(void *p) { delete static_cast<EamState *>(p); }
@@ -309,6 +310,9 @@ static int upload_tables(EamState &st)
     for (int e = 0; e < st.nel; ++e) st.dev.tR[e] = add(st.rho[e]);
     for (int a = 0; a < st.nel; ++a)
         for (int b = 0; b < st.nel; ++b) st.dev.tP[a * EAM_MAX_EL + b] = add(st.phi[a * st.nel + b]);
+    int dev = 0;
+    AGPU_HIP(hipGetDevice(&dev));
+    AGPU_HIP(hipDeviceGetAttribute(&st.ncu, hipDeviceAttributeMultiprocessorCount, dev));
     st.dev.nel = st.nel;
     st.dev.funcfl = st.funcfl ? 1 : 0;
     st.dev.cutoff_sq = st.cutoff * st.cutoff;
@@ -430,27 +434,108 @@ __global__ void k_eam_pack(int nat, const SortedAtom *__restrict__ atoms, const 
     q1[p] = make_double4(a.x, a.y, a.z, (double)el[order[p]]);
 }
 
+// TAB: large single-element systems in FP64 keep the rho table in LDS, as value
+// and scaled curvature z = y'' dx^2 / 6 per knot (16 bytes, so 10 000 knots
+// fit; the coefficients of an interval follow from its two knots:
+// c1 = y1 - y0 - (2 z0 + z1), c2 = 3 z0, c3 = z1 - z0; the errors of energy,
+// forces and virial against the tables' 64-bit sums are those of the general
+// passes to two digits).  The passes are bound by the address
+// processing of their scattered loads, a cache line per lane and load: this
+// takes two of the four loads per neighbour out of the density pass and two of
+// the six out of the force pass (256 000 Cu atoms: density 101 -> 74 us, forces
+// 151 -> 115 us).  One workgroup of 1024 threads per CU walks its share of the
+// atoms.
+constexpr int EAM_TAB = 10180;      // knots: 159 KB of the 160 KB
+constexpr int EAM_TAB_NT = 1024;
+// from 160 atoms per CU: below, filling the table costs more than it saves (both
+// passes together, without and with it: 23 000 atoms 37.6 and 38.0 us, 32 000
+// 44.8 and 44.6, 43 000 56.0 and 54.9, 63 000 77.6 and 66.0, 88 000 99.5 and 86.6)
+constexpr int EAM_TAB_SHARE = 160;
+
+__device__ __forceinline__ void eam_tab_fill(double2 *tab, const SplHdr &h, const double *__restrict__ rec)
+{
+    const double *c = rec + SPL_W * (size_t)h.off;
+    for (int k = threadIdx.x; k < h.n; k += EAM_TAB_NT) {
+        const double *r = c + SPL_W * (size_t)min(k, h.n - 2);
+        // the last knot from the last interval
+        tab[k] = k < h.n - 1 ? make_double2(r[0], r[2] * (1.0 / 3.0))
+                             : make_double2(r[0] + r[1] + r[2] + r[3], r[2] * (1.0 / 3.0) + r[3]);
+    }
+    __syncthreads();
+}
+template <typename R> __device__ __forceinline__ void eam_tab_fill(double2 *, const SplHdr &, const R *) {}
+
+// spl_f and spl_df from the table
+__device__ __forceinline__ double tab_f(const double2 *tab, const SplHdr &h, double x, int &err)
+{
+    double xf;
+    const int i = spl_index(h, x, xf);
+    if (i < 1) {
+        err |= DERR_SPLINE_RANGE;
+        return 1.0;
+    }
+    const double B = xf - i;
+    const double2 a = tab[i - 1], b = tab[i];
+    const double c1 = (b.x - a.x) - (2.0 * a.y + b.y);
+    return a.x + B * (c1 + B * (3.0 * a.y + B * (b.y - a.y)));
+}
+
+__device__ __forceinline__ double tab_df(const double2 *tab, const SplHdr &h, double x, int &err)
+{
+    double xf;
+    const int i = spl_index(h, x, xf);
+    if (i < 1) {
+        err |= DERR_SPLINE_RANGE;
+        return 1.0;
+    }
+    const double B = xf - i;
+    const double2 a = tab[i - 1], b = tab[i];
+    const double c1 = (b.x - a.x) - (2.0 * a.y + b.y);
+    return (c1 + B * (6.0 * a.y + B * (3.0 * (b.y - a.y)))) * h.rdx;
+}
+
+// The atoms of a workgroup: one per lane group, or (TAB) every step'th chunk of
+// APB atoms of its XCD's contiguous share, so that workgroups that run together
+// read neighbouring atoms and dense regions spread over all of them.
+struct EamShare {
+    int first, end, step;
+};
+
+template <bool TAB, int APB> __device__ __forceinline__ EamShare eam_share(int nat)
+{
+    if (!TAB) {
+        const int first = xcd_block() * APB;
+        return {first, min(nat, first + APB), APB};
+    }
+    const int nx = gridDim.x % 8 ? 1 : 8, nw = gridDim.x / nx;
+    const int per = (nat + nx - 1) / nx, x = blockIdx.x % nx;
+    return {x * per + (int)(blockIdx.x / nx) * APB, min(nat, (x + 1) * per), nw * APB};
+}
+
 // KN: one element and every atom tabulated, so no element is read per pair.
-template <typename R, int G, int U, bool ONE, bool KN>
-__global__ void __launch_bounds__(256)
+template <typename R, int G, int U, bool ONE, bool KN, bool TAB>
+__global__ void __launch_bounds__(TAB ? EAM_TAB_NT : 256)
 k_eam_density(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ rec, int nat,
               const int *__restrict__ order, const double4 *__restrict__ q1, CellArg C,
               NlRows L, const int *__restrict__ mask, double4 *__restrict__ q2, double *__restrict__ epa,
               double *__restrict__ partial, int *__restrict__ flags, const int *__restrict__ nlflags)
 {
-    constexpr int APB = 256 / G;
+    constexpr int APB = (TAB ? EAM_TAB_NT : 256) / G;
     __shared__ double s_e[APB];
+    __shared__ __align__(16) double2 tab[TAB ? EAM_TAB : 1];
     // a list build marked unusable: nothing is read from its rows and
     // nothing written but a zero record (the call is redone or refused)
     if (*nlflags & DERR_NL_UNUSABLE) {
         if (threadIdx.x == 0) partial[blockIdx.x] = 0.0;
         return;
     }
+    if (TAB) eam_tab_fill(tab, P.h1R, rec);
     const int lane = threadIdx.x % G, grp = threadIdx.x / G;
-    const int ai = xcd_block() * APB + grp;
-    double Fi = 0.0;
+    const EamShare sh = eam_share<TAB, APB>(nat);
+    double Fsum = 0.0;
     int err = 0;
-    if (ai < nat) {
+    for (int ai = sh.first + grp; ai < sh.end; ai += sh.step) {
+        double Fi = 0.0;
         const int i = order[ai];
         const double4 qi = q1[ai];
         const int eli = KN ? 0 : (int)qi.w;
@@ -481,7 +566,8 @@ k_eam_density(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ re
                     delta_r(C, ri, rj, a, b, c, d);
                     const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
                     if (d2 < P.cutoff_sq)
-                        rho += (double)spl_f<R>(hdr_of<ONE>(P, hdr, 1, elj, 0), rec, sqrt(d2), err);
+                        rho += TAB ? tab_f(tab, P.h1R, sqrt(d2), err)
+                                   : (double)spl_f<R>(hdr_of<ONE>(P, hdr, 1, elj, 0), rec, sqrt(d2), err);
                 }
             }
         }
@@ -498,9 +584,10 @@ k_eam_density(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ re
             q2[ai] = make_double4(qi.x, qi.y, qi.z, dFi);
             if (epa && on) epa[i] += Fi;
         }
+        Fsum += Fi;
     }
     if (err) atomicOr(flags, err);
-    if (lane == 0) s_e[grp] = Fi;
+    if (lane == 0) s_e[grp] = Fsum;
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.0;
@@ -511,29 +598,32 @@ k_eam_density(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ re
 
 // GEN = false: no mask and no per-atom virial requested (the common call),
 // so neither is loaded nor accumulated.
-template <typename R, int G, int U, bool ONE, bool GEN, bool KN>
-__global__ void __launch_bounds__(256)
+template <typename R, int G, int U, bool ONE, bool GEN, bool KN, bool TAB>
+__global__ void __launch_bounds__(TAB ? EAM_TAB_NT : 256)
 k_eam_force(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ rec, int nat,
             const int *__restrict__ order, const double4 *__restrict__ q1, const double4 *__restrict__ q2,
             CellArg C, NlRows L, const int *__restrict__ mask, double *__restrict__ f, double *__restrict__ epa,
             double *__restrict__ wpa, const double *__restrict__ dens_e, double *__restrict__ partial,
             int *__restrict__ flags, const int *__restrict__ nlflags)
 {
-    constexpr int APB = 256 / G;
-    __shared__ double s_red[APB][7];
+    constexpr int NT = TAB ? EAM_TAB_NT : 256, APB = NT / G;
+    // one row of sums per lane group, or (TAB) per wavefront
+    __shared__ double s_red[TAB ? NT / 64 : APB][7];
+    __shared__ __align__(16) double2 tab[TAB ? EAM_TAB : 1];
     if (*nlflags & DERR_NL_UNUSABLE) {
         if (threadIdx.x < 10) partial[(size_t)blockIdx.x * 10 + threadIdx.x] = 0.0;
         return;
     }
+    if (TAB) eam_tab_fill(tab, P.h1R, rec);
     const int lane = threadIdx.x % G, grp = threadIdx.x / G;
-    const int ai = xcd_block() * APB + grp;
-    double acc[3] = {0.0, 0.0, 0.0}, e = 0.0;
+    const EamShare sh = eam_share<TAB, APB>(nat);
+    double esum = 0.0;
     double w[6] = {0, 0, 0, 0, 0, 0};      // own-loop virial (xx yy zz yz xz xy)
-    double wp[6] = {0, 0, 0, 0, 0, 0};     // per-atom virial
     int err = 0;
-    int i = -1;
-    if (ai < nat) {
-        i = order[ai];
+    for (int ai = sh.first + grp; ai < sh.end; ai += sh.step) {
+        double acc[3] = {0.0, 0.0, 0.0}, e = 0.0;
+        double wp[6] = {0, 0, 0, 0, 0, 0};     // per-atom virial
+        const int i = order[ai];
         const int eli = KN ? 0 : (int)q1[ai].w;
         if (eli >= 0) {
             const double mi = (GEN && mask && mask[i] == 0) ? 0.0 : 1.0;
@@ -581,7 +671,8 @@ k_eam_force(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ rec,
                     }
                     const R rr = (R)rrd;
                     const R pp = (dphi - phi * rr) * rr;
-                    const R drho_j = spl_df<R>(hdr_of<ONE>(P, hdr, 1, elj[u], 0), rec, ad, err);
+                    const R drho_j = TAB ? (R)tab_df(tab, P.h1R, ad, err)
+                                         : spl_df<R>(hdr_of<ONE>(P, hdr, 1, elj[u], 0), rec, ad, err);
                     // one element: rho'_i(r) is the same table at the same r
                     const R drho_i = ONE ? drho_j : spl_df<R>(hri, rec, ad, err);
                     const double ci = mi * (double)(dFi * drho_j + pp);
@@ -601,43 +692,46 @@ k_eam_force(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ rec,
                 }
             }
         }
-    }
 #pragma unroll
-    for (int x = 0; x < 3; ++x) acc[x] = group_sum<G>(acc[x]);
-    e = group_sum<G>(e);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) w[q] = group_sum<G>(w[q]);
-    if (GEN && wpa)
-        for (int q = 0; q < 6; ++q) wp[q] = group_sum<G>(wp[q]);
-    if (i >= 0 && lane == 0) {
-        f[3 * (size_t)i] += acc[0];
-        f[3 * (size_t)i + 1] += acc[1];
-        f[3 * (size_t)i + 2] += acc[2];
-        if (epa) epa[i] += e;
-        if (GEN && wpa) {
-            double *o = wpa + 9 * (size_t)i;
-            // column-major 3x3: [a + 3b]
-            o[0] += wp[0];
-            o[4] += wp[1];
-            o[8] += wp[2];
-            o[5] += wp[3];
-            o[7] += wp[3];
-            o[2] += wp[4];
-            o[6] += wp[4];
-            o[1] += wp[5];
-            o[3] += wp[5];
+        for (int x = 0; x < 3; ++x) acc[x] = group_sum<G>(acc[x]);
+        esum += e;
+        if (epa) e = group_sum<G>(e);
+        if (GEN && wpa)
+            for (int q = 0; q < 6; ++q) wp[q] = group_sum<G>(wp[q]);
+        if (lane == 0) {
+            f[3 * (size_t)i] += acc[0];
+            f[3 * (size_t)i + 1] += acc[1];
+            f[3 * (size_t)i + 2] += acc[2];
+            if (epa) epa[i] += e;
+            if (GEN && wpa) {
+                double *o = wpa + 9 * (size_t)i;
+                // column-major 3x3: [a + 3b]
+                o[0] += wp[0];
+                o[4] += wp[1];
+                o[8] += wp[2];
+                o[5] += wp[3];
+                o[7] += wp[3];
+                o[2] += wp[4];
+                o[6] += wp[4];
+                o[1] += wp[5];
+                o[3] += wp[5];
+            }
         }
     }
+    constexpr int SG = TAB ? 64 : G;       // lanes per row of sums
+    esum = group_sum<SG>(esum);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) w[q] = group_sum<SG>(w[q]);
     if (err) atomicOr(flags, err);
-    if (lane == 0) {
-        s_red[grp][0] = e;
-        for (int q = 0; q < 6; ++q) s_red[grp][1 + q] = w[q];
+    if (threadIdx.x % SG == 0) {
+        s_red[threadIdx.x / SG][0] = esum;
+        for (int q = 0; q < 6; ++q) s_red[threadIdx.x / SG][1 + q] = w[q];
     }
     __syncthreads();
     if (threadIdx.x < 7) {
         const int q = threadIdx.x;
         double v = 0.0;
-        for (int k = 0; k < APB; ++k) v += s_red[k][q];
+        for (int k = 0; k < NT / SG; ++k) v += s_red[k][q];
         // record layout [e, W column-major 3x3]; e includes the embedding
         // energy of the same block's atoms from the density pass
         double *rec10 = partial + (size_t)blockIdx.x * 10;
@@ -690,7 +784,7 @@ int eam_bind(agpu_potential *pot)
     return AGPU_OK;
 }
 
-template <typename R, int G, int U, bool ONE, bool GEN, bool KN>
+template <typename R, int G, int U, bool ONE, bool GEN, bool KN, bool TAB = false>
 static int eam_passes(EamState *st, agpu_potential *pot, const agpu_eval_args *a, const R *rec, int nblk)
 {
     agpu_particles *p = pot->p;
@@ -705,11 +799,11 @@ static int eam_passes(EamState *st, agpu_potential *pot, const agpu_eval_args *a
     const int nat = p->nat;
     double4 *q1 = st->pk.as<double4>(), *q2 = q1 + nat;
     const NlRows L = nl_rows(nl);
-    AGPU_LAUNCH(mixed ? "eam_density_mixed" : "eam_density_fp64", (k_eam_density<R, G, U, ONE, KN>), dim3(nblk),
-                dim3(256), 0, s, st->dev, st->d_hdr.as<SplHdr>(), rec, nat, order, q1, C,
+    AGPU_LAUNCH(mixed ? "eam_density_mixed" : "eam_density_fp64", (k_eam_density<R, G, U, ONE, KN, TAB>), dim3(nblk),
+                dim3(TAB ? EAM_TAB_NT : 256), 0, s, st->dev, st->d_hdr.as<SplHdr>(), rec, nat, order, q1, C,
                 L, a->mask, q2, a->epot_per_at, part, flags, nl_flags(nl));
-    AGPU_LAUNCH(mixed ? "eam_force_mixed" : "eam_force_fp64", (k_eam_force<R, G, U, ONE, GEN, KN>), dim3(nblk),
-                dim3(256), 0, s, st->dev, st->d_hdr.as<SplHdr>(), rec, nat, order, q1, q2, C,
+    AGPU_LAUNCH(mixed ? "eam_force_mixed" : "eam_force_fp64", (k_eam_force<R, G, U, ONE, GEN, KN, TAB>), dim3(nblk),
+                dim3(TAB ? EAM_TAB_NT : 256), 0, s, st->dev, st->d_hdr.as<SplHdr>(), rec, nat, order, q1, q2, C,
                 L, a->mask, a->f, a->epot_per_at, a->wpot_per_at, part, part + nblk, flags, nl_flags(nl));
     return AGPU_OK;
 }
@@ -753,6 +847,12 @@ static int eam_launch(EamState *st, agpu_potential *pot, const agpu_eval_args *a
             case 3202: return eam_passes<R, 32, 2, ONE, false, KN>(st, pot, a, rec, nblk);
             case 3204: return eam_passes<R, 32, 4, ONE, false, KN>(st, pot, a, rec, nblk);
             default: break;
+            }
+            if constexpr (sizeof(R) == 8 && EAM_G == 16 && EAM_U == 4) {
+                if (st->dev.h1R.n <= EAM_TAB && nat >= EAM_TAB_SHARE * st->ncu) {
+                    *nblk_out = st->ncu;
+                    return eam_passes<R, EAM_G, EAM_U, ONE, false, KN, true>(st, pot, a, rec, st->ncu);
+                }
             }
         }
     }

@@ -217,6 +217,37 @@ def _close(a, b, rel=1e-10):
     return np.abs(a - b).max() <= rel * max(1.0, np.abs(b).max())
 
 
+@pytest.mark.parametrize("n,slab", [((21, 21, 23), False), ((22, 22, 22), True), ((24, 25, 26), False)])
+def test_eam_table_in_lds(n, slab):
+    """From 160 atoms per CU (40 960) the FP64 passes read the density table
+    from LDS; a call with per-atom virials keeps the general passes.  Sizes: just
+    below, above with remainders in every share, and a slab (an uneven one).
+    Two roundings per pair and 54 pairs with both signs per force: 1e-12 of the
+    largest force, as between the tuned variants."""
+    a = 3.615
+    cells = np.stack(np.meshgrid(*[np.arange(k) for k in n], indexing="ij"), -1).reshape(-1, 1, 3)
+    base = np.array([[0, 0, 0], [0, .5, .5], [.5, 0, .5], [.5, .5, 0]])
+    pos = ((cells + base) * a).reshape(-1, 3)
+    pos = pos + np.random.default_rng(5).normal(0, 0.08, pos.shape)
+    cell = np.diag(np.array(n) * a)
+    if slab:
+        cell[2, 2] *= 2.0
+    p = N.from_atoms(pos, cell, np.array([True, True, not slab]), np.full(len(pos), 29, np.int32))
+    nl = N.Neighbors(100)
+    pot = N.TabulatedAlloyEAM(fn=MISHIN)
+    pot.bind_to(p, nl)
+    e0, f0, w0, epa0, *_ = pot.energy_and_forces(p, nl, epot_per_at=True, wpot_per_at=True)
+    e, f, w, epa, *_ = pot.energy_and_forces(p, nl, epot_per_at=True)
+    e2, f2, w2, *_ = pot.energy_and_forces(p, nl)
+    assert abs(e - e0) <= 1e-13 * abs(e0)
+    assert np.abs(f - f0).max() <= 1e-12 * np.abs(f0).max()
+    # the virial's terms cancel between repulsion and attraction
+    scale = (np.abs(f0) * a * 3).sum()
+    assert np.abs(w - w0).max() <= 1e-13 * scale
+    assert np.abs(epa - epa0).max() <= 1e-13 * np.abs(epa0).max()
+    assert e2 == e and np.array_equal(f2, f) and np.array_equal(w2, w)
+
+
 def test_eam_deferred_list_check_redo():
     """EAM checks its list build's flags with its own at the end of the call.
     A build that outgrew the staging stride, and one whose crowded bin hands
