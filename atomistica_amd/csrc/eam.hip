@@ -61,6 +61,7 @@ struct HostSpline {
 };
 
 constexpr int SPL_W = 4;       // coefficients per interval record
+constexpr int EAM_TAB = 10180; // knots of a table kept in LDS: 159 KB of its 160 KB
 
 static void spline_build(HostSpline &s, const std::vector<double> &y, double dx, double scale)
 {
@@ -109,6 +110,7 @@ struct EamDev {
     int tF[EAM_MAX_EL], tR[EAM_MAX_EL], tP[EAM_MAX_EL * EAM_MAX_EL];
     double cutoff_sq;
     SplHdr h1F, h1R, h1P;     // the three tables of a single-element potential
+    const double2 *knots;     // rho's knots behind the 64-bit records, or null
 };
 
 struct EamState {
@@ -320,8 +322,18 @@ static int upload_tables(EamState &st)
     st.dev.h1R = st.hdr[st.dev.tR[0]];
     st.dev.h1P = st.hdr[st.dev.tP[0]];
     std::vector<float> rec32(rec64.begin(), rec64.end());
+    // the knots of rho (value, c2 / 3) behind the records, as the passes with
+    // the table in LDS copy them; the last from the last interval
+    const std::vector<double> &c = st.rho[0].rec;
+    const size_t knots = rec64.size();
+    if (st.nel == 1 && !c.empty() && st.rho[0].n <= EAM_TAB) {
+        for (size_t k = 0; k < c.size(); k += SPL_W) rec64.insert(rec64.end(), {c[k], c[k + 2] / 3.0});
+        const double *l = &c[c.size() - SPL_W];
+        rec64.insert(rec64.end(), {l[0] + l[1] + l[2] + l[3], l[2] / 3.0 + l[3]});
+    }
     AGPU_CHECK(st.d_hdr.reserve(sizeof(SplHdr) * st.hdr.size()));
     AGPU_CHECK(st.d_rec64.reserve(sizeof(double) * rec64.size()));
+    st.dev.knots = rec64.size() > knots ? (const double2 *)(st.d_rec64.as<double>() + knots) : nullptr;
     AGPU_CHECK(st.d_rec32.reserve(sizeof(float) * rec32.size()));
     hipStream_t s = stream();
     AGPU_HIP(hipMemcpyAsync(st.d_hdr.ptr, st.hdr.data(), sizeof(SplHdr) * st.hdr.size(), hipMemcpyHostToDevice, s));
@@ -434,36 +446,30 @@ __global__ void k_eam_pack(int nat, const SortedAtom *__restrict__ atoms, const 
     q1[p] = make_double4(a.x, a.y, a.z, (double)el[order[p]]);
 }
 
-// TAB: large single-element systems in FP64 keep the rho table in LDS, as value
-// and scaled curvature z = y'' dx^2 / 6 per knot (16 bytes, so 10 000 knots
-// fit; the coefficients of an interval follow from its two knots:
-// c1 = y1 - y0 - (2 z0 + z1), c2 = 3 z0, c3 = z1 - z0; the errors of energy,
-// forces and virial against the tables' 64-bit sums are those of the general
-// passes to two digits).  The passes are bound by the address
-// processing of their scattered loads, a cache line per lane and load: this
-// takes two of the four loads per neighbour out of the density pass and two of
-// the six out of the force pass (256 000 Cu atoms: density 101 -> 74 us, forces
-// 151 -> 115 us).  One workgroup of 1024 threads per CU walks its share of the
+// TAB: large single-element systems keep the rho table in LDS, as value and
+// scaled curvature z = y'' dx^2 / 6 per knot (16 bytes, so 10 000 knots fit;
+// the coefficients of an interval follow from its two knots:
+// c1 = y1 - y0 - (2 z0 + z1), c2 = 3 z0, c3 = z1 - z0; the FP64 errors of
+// energy, forces and virial are those of the general passes to two digits).
+// In FP64 in both precisions: differences of knots lose digits in FP32.
+// The passes are bound by the address processing of their scattered loads, a
+// cache line per lane and load: this takes two of the four loads per neighbour
+// out of the density pass and two of the six out of the force pass (256 000 Cu
+// atoms: density 101 -> 74 us, forces 151 -> 115 us; mixed 77 -> 74 and
+// 126 -> 101 us).  One workgroup of 1024 threads per CU walks its share of the
 // atoms.
-constexpr int EAM_TAB = 10180;      // knots: 159 KB of the 160 KB
 constexpr int EAM_TAB_NT = 1024;
-// from 160 atoms per CU: below, filling the table costs more than it saves (both
-// passes together, without and with it: 23 000 atoms 37.6 and 38.0 us, 32 000
-// 44.8 and 44.6, 43 000 56.0 and 54.9, 63 000 77.6 and 66.0, 88 000 99.5 and 86.6)
-constexpr int EAM_TAB_SHARE = 160;
+// Atoms per CU from which it is taken: with fewer, filling the table costs more
+// than it saves.  Both passes together, without and with it: FP64 23 000 atoms
+// 37.6 and 38.0 us, 43 000 56.0 and 52.5, 63 000 77.6 and 65.1; mixed 43 000
+// 48.9 and 50.6, 63 000 66.0 and 61.7.
+template <typename R> constexpr int eam_tab_share() { return sizeof(R) == 8 ? 160 : 220; }
 
-__device__ __forceinline__ void eam_tab_fill(double2 *tab, const SplHdr &h, const double *__restrict__ rec)
+__device__ __forceinline__ void eam_tab_fill(double2 *tab, int n, const double2 *__restrict__ knots)
 {
-    const double *c = rec + SPL_W * (size_t)h.off;
-    for (int k = threadIdx.x; k < h.n; k += EAM_TAB_NT) {
-        const double *r = c + SPL_W * (size_t)min(k, h.n - 2);
-        // the last knot from the last interval
-        tab[k] = k < h.n - 1 ? make_double2(r[0], r[2] * (1.0 / 3.0))
-                             : make_double2(r[0] + r[1] + r[2] + r[3], r[2] * (1.0 / 3.0) + r[3]);
-    }
+    for (int k = threadIdx.x; k < n; k += EAM_TAB_NT) tab[k] = knots[k];
     __syncthreads();
 }
-template <typename R> __device__ __forceinline__ void eam_tab_fill(double2 *, const SplHdr &, const R *) {}
 
 // spl_f and spl_df from the table
 __device__ __forceinline__ double tab_f(const double2 *tab, const SplHdr &h, double x, int &err)
@@ -529,7 +535,7 @@ k_eam_density(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ re
         if (threadIdx.x == 0) partial[blockIdx.x] = 0.0;
         return;
     }
-    if (TAB) eam_tab_fill(tab, P.h1R, rec);
+    if (TAB) eam_tab_fill(tab, P.h1R.n, P.knots);
     const int lane = threadIdx.x % G, grp = threadIdx.x / G;
     const EamShare sh = eam_share<TAB, APB>(nat);
     double Fsum = 0.0;
@@ -614,7 +620,7 @@ k_eam_force(EamDev P, const SplHdr *__restrict__ hdr, const R *__restrict__ rec,
         if (threadIdx.x < 10) partial[(size_t)blockIdx.x * 10 + threadIdx.x] = 0.0;
         return;
     }
-    if (TAB) eam_tab_fill(tab, P.h1R, rec);
+    if (TAB) eam_tab_fill(tab, P.h1R.n, P.knots);
     const int lane = threadIdx.x % G, grp = threadIdx.x / G;
     const EamShare sh = eam_share<TAB, APB>(nat);
     double esum = 0.0;
@@ -848,8 +854,8 @@ static int eam_launch(EamState *st, agpu_potential *pot, const agpu_eval_args *a
             case 3204: return eam_passes<R, 32, 4, ONE, false, KN>(st, pot, a, rec, nblk);
             default: break;
             }
-            if constexpr (sizeof(R) == 8 && EAM_G == 16 && EAM_U == 4) {
-                if (st->dev.h1R.n <= EAM_TAB && nat >= EAM_TAB_SHARE * st->ncu) {
+            if constexpr (EAM_G == 16 && EAM_U == 4) {
+                if (st->dev.knots && nat >= eam_tab_share<R>() * st->ncu) {
                     *nblk_out = st->ncu;
                     return eam_passes<R, EAM_G, EAM_U, ONE, false, KN, true>(st, pot, a, rec, st->ncu);
                 }

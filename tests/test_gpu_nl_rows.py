@@ -219,9 +219,9 @@ def _close(a, b, rel=1e-10):
 
 @pytest.mark.parametrize("n,slab", [((21, 21, 23), False), ((22, 22, 22), True), ((24, 25, 26), False)])
 def test_eam_table_in_lds(n, slab):
-    """From 160 atoms per CU (40 960) the FP64 passes read the density table
-    from LDS; a call with per-atom virials keeps the general passes.  Sizes: just
-    below, above with remainders in every share, and a slab (an uneven one).
+    """From 160 atoms per CU (40 960; mixed 56 320) the passes read the density
+    table from LDS; a call with per-atom virials keeps the general passes.
+    Sizes: just below, above with remainders in every share, and a slab.
     Two roundings per pair and 54 pairs with both signs per force: 1e-12 of the
     largest force, as between the tuned variants."""
     a = 3.615
@@ -246,6 +246,11 @@ def test_eam_table_in_lds(n, slab):
     assert np.abs(w - w0).max() <= 1e-13 * scale
     assert np.abs(epa - epa0).max() <= 1e-13 * np.abs(epa0).max()
     assert e2 == e and np.array_equal(f2, f) and np.array_equal(w2, w)
+    # FP32 pair arithmetic: a force is a sum of 54 terms of up to a few eV/A
+    pot.set_precision("mixed")
+    em, fm, wm, *_ = pot.energy_and_forces(p, nl)
+    assert abs(em - e0) <= 1e-7 * abs(e0)
+    assert np.abs(fm - f0).max() <= 54 * 2.0 ** -23 * np.abs(f0).max()
 
 
 def test_eam_deferred_list_check_redo():
