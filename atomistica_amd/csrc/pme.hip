@@ -35,6 +35,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "agpu_internal.hpp"
+#include "pme_cell.hpp"
 #include "profile.hpp"
 
 namespace agpu {
@@ -89,24 +90,6 @@ __host__ __device__ __forceinline__ void fill_bspline(double w, int order, doubl
     d[0] = -c[0];
     for (int j = 1; j < order; ++j) d[j] = c[j - 1] - c[j];
     bsp_one_pass(c, w, order);
-}
-
-__device__ __forceinline__ int wrapi(int x, int K) { return ((x % K) + K) % K; }
-
-struct PmeGrid {
-    int K[3], nb[3];     // points and bricks per axis
-};
-
-// scaled fractional of one axis: wrapped grid cell ib and the offset in it
-__device__ __forceinline__ double pme_cell(const CellArg &B, const PmeGrid &g, int e, double x, double y, double z,
-                                           int &ib)
-{
-    // w = x recip(1,e) + y recip(2,e) + z recip(3,e)  (get_scaled_fractionals)
-    const double w = x * B.A[0 + 3 * e] + y * B.A[1 + 3 * e] + z * B.A[2 + 3 * e];
-    const double fr = g.K[e] * (w - round(w) + 0.5);
-    const int i = (int)fr;
-    ib = wrapi(i, g.K[e]);
-    return fr - i;
 }
 
 // cnt (counting sort): the ion's provisional place in its brick; else its

@@ -118,3 +118,25 @@ def test_pme_brick_edges(n, grid, order, shear):
     e, f, w, phi = gpu(pos, q, cell, [True] * 3, Z, 4.0, grid, order)
     assert abs(e - e0) <= REL * max(1.0, abs(e0))
     assert close(f, f0) and close(w, w0) and close(phi, p0)
+
+
+@pytest.mark.parametrize("grid,order", [((16, 24, 40), 4), ((16, 24, 40), 8), ((41, 17, 24), 6)])
+def test_pme_ions_on_brick_faces(grid, order):
+    """Ions on the faces of bricks of 8^3 grid cells, or one ulp of a
+    coordinate to either side, in a sheared cell and around it: the brick that
+    an ion is sorted into and the place of its points there agree."""
+    rng = np.random.default_rng(sum(grid))
+    cell = np.diag([9.0, 10.0, 12.0]) @ (np.eye(3) + 0.15 * np.array([[0, 1, 0.5], [1, 0, -0.4], [0.5, -0.4, 0]]))
+    n, K = 200, np.array(grid)
+    frac = rng.integers(0, 1 + K // 8, (n, 3)) * 8.0 / K - 0.5 + rng.integers(-1, 2, (n, 3))
+    frac[np.arange(n), rng.integers(0, 3, n)] = rng.random(n)
+    pos = frac @ cell
+    for step in (-np.inf, np.inf):
+        pos = np.where(rng.random(pos.shape) < 0.25, np.nextafter(pos, step), pos)
+    q = rng.normal(size=n)
+    q -= q.mean()
+    print("pme brick faces", grid, order, flush=True)
+    e0, f0, w0, p0 = oracle(pos, q, cell, [True] * 3, 4.0, grid, order)
+    e, f, w, phi = gpu(pos, q, cell, [True] * 3, np.full(n, 11, np.int32), 4.0, grid, order)
+    assert abs(e - e0) <= REL * max(1.0, abs(e0))
+    assert close(f, f0) and close(w, w0) and close(phi, p0)
