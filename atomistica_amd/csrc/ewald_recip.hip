@@ -356,8 +356,8 @@ __device__ __forceinline__ void ewr_force_steps(const double2 *__restrict__ uvp,
 // multiplies while the other applies its column phases (one workgroup of
 // eight waves left the matrix cores idle there).
 __global__ void __launch_bounds__(64 * EWR_FW, 2)
-k_ewr_force(const EwrFBlock *__restrict__ blks, const EwrItem *__restrict__ items, int nat,
-            const double4 *__restrict__ s4, const double2 *__restrict__ T, double4 *__restrict__ part)
+k_ewr_force(const EwrFBlock *__restrict__ blks, const EwrItem *__restrict__ items, const double4 *__restrict__ s4,
+            const double2 *__restrict__ T, double4 *__restrict__ part)
 {
     __shared__ __align__(16) double2 sT[2][EWR_FT * 256];
     const EwrFBlock B = blks[blockIdx.x];
@@ -431,23 +431,23 @@ k_ewr_force(const EwrFBlock *__restrict__ blks, const EwrItem *__restrict__ item
         a3 += __shfl_xor(a3, o, 64);
         ap += __shfl_xor(ap, o, 64);
     }
-    if (act && lane < 16) part[(size_t)B.split * nat + j] = make_double4(a1, a2, a3, ap);
+    if (act && lane < 16) part[B.rec + j] = make_double4(a1, a2, a3, ap);
 }
 
-// f += q E and phi += phi_rec from the ions' partial sums (nsplit of them, or
-// the number that the ion's structure has)
-__global__ void k_ewr_apply(int nat, int nsplit, const int *__restrict__ sof, const int *__restrict__ fsplit,
+// f += q E and phi += phi_rec from the ions' partial sums, as many as the ion's
+// structure has splits
+__global__ void k_ewr_apply(int nat, const int *__restrict__ sof, const EwrFRec *__restrict__ frec,
                             const double *__restrict__ geo, const double4 *__restrict__ s4,
                             const double4 *__restrict__ part, double *__restrict__ f, double *__restrict__ phi)
 {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= nat) return;
     const int s = sof ? sof[j] : 0;
-    const int n = sof ? fsplit[s] : nsplit;
+    const EwrFRec R = frec[s];
     const double *G = geo + EWR_GEO * (size_t)s;
     double a1 = 0.0, a2 = 0.0, a3 = 0.0, ap = 0.0;
-    for (int k = 0; k < n; ++k) {
-        const double4 v = part[(size_t)k * nat + j];
+    for (int k = 0; k < R.nsplit; ++k) {
+        const double4 v = part[R.rec + (long long)k * R.n + j];
         a1 += v.x;
         a2 += v.y;
         a3 += v.z;
@@ -528,7 +528,8 @@ int ewr_plan(EwrState &st, int ns, const double *cells, const int *off, double k
     st.fblk.clear();
     st.tile0.assign(ns + 1, 0);
     std::vector<double> geo((size_t)EWR_GEO * ns, 0.0);
-    std::vector<int> item0(ns + 1, 0), fsplit(ns, 1);
+    std::vector<int> item0(ns + 1, 0);
+    std::vector<EwrFRec> frec(ns);
     std::vector<int2> map;
     long long tiles = 0, stiles = 0, swork = 0, fwork = 0;
     for (int s = 0; s < ns; ++s) {
@@ -571,14 +572,12 @@ int ewr_plan(EwrState &st, int ns, const double *cells, const int *off, double k
     // (512 of either), but no less than costs its set-up.
     const long long starget = std::max(swork / (EWR_SW * 512ll * 12), 64ll * 2);
     const long long ftarget = std::max(fwork / (512ll * 12), 24ll);
-    st.nfsplit = 1;
+    st.nfrec = 0;
     for (int s = 0; s < ns; ++s) {
         const int a0 = off[s], n = off[s + 1] - off[s];
         const int nt_s = st.tile0[s + 1] - st.tile0[s];
-        if (nt_s == 0) {
-            fsplit[s] = 0;
-            continue;
-        }
+        frec[s] = EwrFRec{0, n, 0};
+        if (nt_s == 0) continue;
         // splits of the ions: by the structure's largest item, whole LDS chunks
         int ntm = 1;
         long long fw = 0;
@@ -623,11 +622,13 @@ int ewr_plan(EwrState &st, int ns, const double *cells, const int *off, double k
         }
         nf = (int)cut.size();
         cut.push_back(item0[s + 1]);
-        fsplit[s] = nf;
-        st.nfsplit = std::max(st.nfsplit, nf);
+        frec[s].nsplit = nf;
+        frec[s].rec = st.nfrec - a0;
+        st.nfrec += (long long)nf * n;
         for (int sp = 0; sp < nf; ++sp)
             for (int a = 0; a < n; a += EWR_FI)
-                st.fblk.push_back(EwrFBlock{a0 + a, std::min(a0 + n, a0 + a + EWR_FI), cut[sp], cut[sp + 1], sp, 0, 0, 0});
+                st.fblk.push_back(EwrFBlock{a0 + a, std::min(a0 + n, a0 + a + EWR_FI), cut[sp], cut[sp + 1],
+                                            frec[s].rec + (long long)sp * n, 0});
     }
     // the longest workgroups first
     auto fcost = [&](const EwrFBlock &x) {
@@ -647,9 +648,8 @@ int ewr_plan(EwrState &st, int ns, const double *cells, const int *off, double k
     AGPU_CHECK(ewr_upload(st.d_fblk, st.fblk, hs));
     AGPU_CHECK(ewr_upload(st.d_map, map, hs));
     AGPU_CHECK(ewr_upload(st.d_geo, geo, hs));
-    std::vector<int> tf(st.tile0);
-    tf.insert(tf.end(), fsplit.begin(), fsplit.end());
-    AGPU_CHECK(ewr_upload(st.d_tile0, tf, hs));
+    AGPU_CHECK(ewr_upload(st.d_frec, frec, hs));
+    AGPU_CHECK(ewr_upload(st.d_tile0, st.tile0, hs));
     AGPU_CHECK(st.S.reserve(sizeof(double) * 512 * (size_t)(stiles + 1)));
     AGPU_CHECK(st.T.reserve(sizeof(double2) * 256 * (size_t)(tiles + 1)));
     AGPU_HIP(hipStreamSynchronize(hs));
@@ -671,12 +671,11 @@ int ewr_run(EwrState &st, int nat, const double *r, const double *q, const int *
     AGPU_LAUNCH("ewald_kenergy", k_ewr_energy, dim3(st.ntile), dim3(128), 0, s, st.d_map.as<int2>(), items, geo,
                 kmax * kmax, 1.0 / (4.0 * beta * beta), st.S.as<double>(), st.T.as<double2>(), rec);
     if (!f && !phi) return AGPU_OK;
-    AGPU_CHECK(st.fpart.reserve(sizeof(double4) * (size_t)nat * st.nfsplit));
+    AGPU_CHECK(st.fpart.reserve(sizeof(double4) * (size_t)st.nfrec));
     AGPU_LAUNCH("ewald_kforce", k_ewr_force, dim3((unsigned)st.fblk.size()), dim3(64 * EWR_FW), 0, s,
-                st.d_fblk.as<EwrFBlock>(), items, nat, s4, st.T.as<double2>(), st.fpart.as<double4>());
-    const int ns = (int)st.tile0.size() - 1;
-    AGPU_LAUNCH("ewald_kapply", k_ewr_apply, dim3((nat + 255) / 256), dim3(256), 0, s, nat, st.nfsplit, sof,
-                st.d_tile0.as<int>() + ns + 1, geo, s4, st.fpart.as<double4>(), f, phi);
+                st.d_fblk.as<EwrFBlock>(), items, s4, st.T.as<double2>(), st.fpart.as<double4>());
+    AGPU_LAUNCH("ewald_kapply", k_ewr_apply, dim3((nat + 255) / 256), dim3(256), 0, s, nat, sof,
+                st.d_frec.as<EwrFRec>(), geo, s4, st.fpart.as<double4>(), f, phi);
     return AGPU_OK;
 }
 

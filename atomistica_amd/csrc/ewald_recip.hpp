@@ -25,19 +25,28 @@ struct EwrSBlock {
     int item, nitem, a0, a1, split, t0, nt, pad;
 };
 
-// forces: one workgroup: ions [a0, a1) of one structure, items [i0, i1)
+// forces: one workgroup: ions [a0, a1) of one structure, items [i0, i1); ion
+// j's partial sums go to record rec + j
 struct EwrFBlock {
-    int a0, a1, i0, i1, split, pad0, pad1, pad2;
+    int a0, a1, i0, i1;
+    long long rec, pad;
+};
+
+// where the partial sums of a structure's forces are: those of ion j and split
+// k < nsplit are record rec + k n + j
+struct EwrFRec {
+    long long rec;
+    int n, nsplit;
 };
 
 struct EwrState {
     int ntile = 0;       // tiles of T (and records)
-    int nfsplit = 0;     // partial force records per ion (largest over the structures)
+    long long nfrec = 0; // partial force records, each structure's ions times its splits
     std::vector<EwrItem> items;
     std::vector<EwrSBlock> sblk;
     std::vector<EwrFBlock> fblk;
     std::vector<int> tile0;   // first tile of each structure (nstruct + 1)
-    DevBuf d_items, d_sblk, d_fblk, d_map, d_geo, d_tile0, S, T, s4, fpart;
+    DevBuf d_items, d_sblk, d_fblk, d_frec, d_map, d_geo, d_tile0, S, T, s4, fpart;
 };
 
 // Patches, tiles and work blocks for structures with cells[9 s + 3 k + x] =

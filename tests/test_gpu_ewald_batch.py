@@ -135,3 +135,35 @@ def test_ewald_batch_256_cells():
         re_, rf, _, _ = _oracle(pos, cell, q[a0:a1], beta, kmax)
         assert abs(float(e1[s]) - re_) <= REL * abs(re_)
         assert _close(fn[a0:a1], rf)
+
+
+def test_wide_cell_does_not_grow_the_scratch_of_others():
+    """200 cells of 512 ions and one of 100 A with 64: the wide cell's k are
+    shared out over many workgroups.  The partial forces of each cell take the
+    splits of that cell only, so a call with forces needs little more memory
+    than one without: 32 bytes per ion and split, in all 64 ions x 6144
+    workgroups and two more splits per ion.  The wide cell matches the oracle."""
+    import torch
+    from atomistica_amd.batch import Batch, ewald_batch
+    beta, kmax = _params()
+    S, q = W.rocksalt_cells(200, nmin=4, nmax=4)
+    n = sum(len(p) for p, _ in S)
+    rng = np.random.default_rng(8)
+    cell = np.diag([100.0, 100.0, 100.0])
+    pos = rng.random((64, 3)) @ cell
+    qw = np.where(np.arange(64) % 2, 1.0, -1.0)
+    b = Batch(S + [(pos, cell)])
+    q = np.concatenate([q, qw])
+    print("ewald batch with a wide cell", n + 64, flush=True)
+    ewald_batch(b, q, RC, beta, kmax, forces=False, virial=False)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    e, f, w, phi = ewald_batch(b, q, RC, beta, kmax, phi=True)
+    torch.cuda.synchronize()
+    grown = before - torch.cuda.mem_get_info()[0]
+    print("  a call with forces takes %.1f MB more" % (grown / 1e6), flush=True)
+    # the partial forces, and torch's blocks of the returned arrays
+    assert grown <= 32 * (64 * 6144 + 2 * (n + 64)) + 64e6
+    e0, f0, w0, p0 = _oracle(pos, cell, qw, beta, kmax)
+    assert abs(e[-1].item() - e0) <= REL * abs(e0)
+    assert _close(f[-64:].cpu(), f0) and _close(w[-1].cpu(), w0) and _close(phi[-64:].cpu(), p0)
