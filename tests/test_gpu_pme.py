@@ -140,3 +140,37 @@ def test_pme_ions_on_brick_faces(grid, order):
     e, f, w, phi = gpu(pos, q, cell, [True] * 3, np.full(n, 11, np.int32), 4.0, grid, order)
     assert abs(e - e0) <= REL * max(1.0, abs(e0))
     assert close(f, f0) and close(w, w0) and close(phi, p0)
+
+
+@pytest.mark.parametrize("n", [60, 64, 65, 300, 2000, 20000])
+def test_pme_cluster_in_one_brick(n):
+    """n ions of a salt cluster in one brick and 40 more anywhere in the cell:
+    the brick's ions are put into index order by comparing them, or, where that
+    grows with the square, from the keys of all ions (n above 64).  20 000 ions
+    in one brick take 306 ms by comparing and 0.035 ms by the walk."""
+    rng = np.random.default_rng(n)
+    grid, L = (64, 64, 64), 800.0
+    m = int(np.ceil(n ** (1 / 3)))
+    site = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    pos = 105.0 + 2.82 * site + rng.uniform(-0.2, 0.2, (n, 3))
+    q = np.where(site.sum(1) % 2, 1.0, -1.0)
+    assert pos.max() < 200.0                     # the brick from 100 to 200 A
+    pos = np.concatenate([pos, rng.random((40, 3)) * L])
+    q = np.concatenate([q, rng.normal(size=40)])
+    perm = rng.permutation(n + 40)
+    pos, q = pos[perm], (q - q.mean())[perm]
+    cell = np.diag([L, L, L])
+    Z = np.full(n + 40, 11, np.int32)
+    print("pme cluster", n, flush=True)
+    e0, f0, w0, p0 = oracle(pos, q, cell, [True] * 3, 4.0, grid, 4)
+    N.profile_enable(True)
+    N.profile_reset()
+    e, f, w, phi = gpu(pos, q, cell, [True] * 3, Z, 4.0, grid, 4)
+    ms, calls = N.profile_query("pme_order")
+    N.profile_enable(False)
+    print("  pme_order %.3f ms" % (ms / calls), flush=True)
+    assert abs(e - e0) <= REL * max(1.0, abs(e0))
+    assert close(f, f0) and close(w, w0) and close(phi, p0)
+    assert ms / calls < 20.0
+    again = gpu(pos, q, cell, [True] * 3, Z, 4.0, grid, 4)
+    assert e == again[0] and np.array_equal(f, again[1]) and np.array_equal(phi, again[3])
