@@ -12,7 +12,7 @@
 //   fc = trig_off on [R, S] (cutoff.f90:171-196).
 //
 // Kernels:
-//   k_bnl<false> / k_bnl<true>  wavefront per atom: every periodic image of
+//   k_bnl<false> / k_bnl<true>  lane group per atom: every periodic image of
 //       every atom of the same structure with |r_i - r_j + A n|^2 < S^2 (the
 //       image range per axis from the reciprocal vectors), counted, scanned,
 //       then written in (j ascending, n lexicographic) order together with
@@ -103,31 +103,32 @@ int batch_fractions(agpu_batch *b)
     return AGPU_OK;
 }
 
-// A wavefront per atom: 64 atoms of its structure at a time, a lane each.  A
+// G lanes per atom: G atoms of its structure at a time, a lane each.  A
 // lane screens its atom's images in FP32 (the nearest one, and those around it
 // in cells below twice the cut-off), takes the FP64 test for what is left,
 // and the lanes' counts place its entries, so a row keeps its order (j
-// ascending, images lexicographic).  4096 Si structures (494 801 atoms): the
-// two passes took 10.9 ms with a thread per atom that bounded the images of
-// every pair in FP64, and take 1.65 ms.
-template <bool FILL>
+// ascending, images lexicographic); a single lane writes as it goes.  4096 Si
+// structures (494 801 atoms): the two passes took 10.9 ms with a thread per
+// atom that bounded the images of every pair in FP64, and take 1.65 ms.
+template <bool FILL, int G>
 __global__ void __launch_bounds__(256)
-k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, StructGeom G, double rc,
+k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, StructGeom SG, double rc,
       const int *__restrict__ offsets, int *__restrict__ counts, int2 *__restrict__ nbr, int *__restrict__ own,
       double4 *__restrict__ bnd64, float4 *__restrict__ bnd32, int *__restrict__ flags)
 {
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & (G - 1);
+    const int sub = threadIdx.x / G;
+    const int i = blockIdx.x * (256 / G) + (G == 64 ? __builtin_amdgcn_readfirstlane(sub) : sub);
     if (i >= ntot) return;
-    const int s = G.sof[i];
-    const int a0 = G.off[s], a1 = G.off[s + 1];
+    const int s = SG.sof[i];
+    const int a0 = SG.off[s], a1 = SG.off[s + 1];
     CellArg C;
     double b[9];
     float Af[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) {
-        C.A[q] = G.cell[9 * (size_t)s + q];
-        b[q] = G.rec[9 * (size_t)s + q];
+        C.A[q] = SG.cell[9 * (size_t)s + q];
+        b[q] = SG.rec[9 * (size_t)s + q];
         Af[q] = (float)C.A[q];
     }
     int m[3];
@@ -137,7 +138,7 @@ k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, Struct
     const int4 ui = u[i];
     int total = FILL ? offsets[i] : 0;
     bool bad = false;
-    for (int base = a0; base < a1; base += 64) {
+    for (int base = a0; base < a1; base += G) {
         const int j = base + lane;
         int du[3];
         batch_diff(ui, u[min(j, a1 - 1)], du);
@@ -146,6 +147,20 @@ k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, Struct
         double rj[3] = {0.0, 0.0, 0.0};
         int near[3] = {0, 0, 0};        // the nearest image
         bool loaded = false;
+        auto load = [&]() {
+            loaded = true;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) rj[k] = r[3 * (size_t)j + k];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                // the whole turns between the difference and its wrapped form
+                const double ds = b[3 * k] * (ri[0] - rj[0]) + b[3 * k + 1] * (ri[1] - rj[1]) +
+                                  b[3 * k + 2] * (ri[2] - rj[2]);
+                near[k] = (int)rint((double)du[k] * BATCH_TURN - ds);
+            }
+        };
+        // nearly every atom of a small structure has an image in reach
+        if (G < 64 && j < a1) load();
         // visits the accepted images in order
         auto images = [&](auto &&visit) {
             for (int o0 = -m[0]; o0 <= m[0]; ++o0)
@@ -156,18 +171,7 @@ k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, Struct
                         const float y = Af[1] * v0 + Af[4] * v1 + Af[7] * v2;
                         const float z = Af[2] * v0 + Af[5] * v1 + Af[8] * v2;
                         if (j >= a1 || !(x * x + y * y + z * z < rs2)) continue;
-                        if (!loaded) {
-                            loaded = true;
-#pragma unroll
-                            for (int k = 0; k < 3; ++k) rj[k] = r[3 * (size_t)j + k];
-#pragma unroll
-                            for (int k = 0; k < 3; ++k) {
-                                // the whole turns between the difference and its wrapped form
-                                const double ds = b[3 * k] * (ri[0] - rj[0]) + b[3 * k + 1] * (ri[1] - rj[1]) +
-                                                  b[3 * k + 2] * (ri[2] - rj[2]);
-                                near[k] = (int)rint((double)du[k] * BATCH_TURN - ds);
-                            }
-                        }
+                        if (!loaded) load();
                         const int n0 = near[0] + o0, n1 = near[1] + o1, n2 = near[2] + o2;
                         if (j == i && n0 == 0 && n1 == 0 && n2 == 0) continue;
                         double d[3];
@@ -181,32 +185,39 @@ k_bnl(int ntot, const double *__restrict__ r, const int4 *__restrict__ u, Struct
                         visit(n0, n1, n2, d, d2);
                     }
         };
+        auto write = [&](size_t at, int n0, int n1, int n2, const double *d, double d2) {
+            // bond i -> image of j: r_ij = -d, unit vector -d / |d|
+            const double l = sqrt(d2);
+            const double u0 = -d[0] / l, u1 = -d[1] / l, u2 = -d[2] / l;
+            nbr[at] = make_int2(j, dc_pack(n0, n1, n2));
+            own[at] = i;
+            bnd64[at] = make_double4(u0, u1, u2, l);
+            bnd32[at] = make_float4((float)u0, (float)u1, (float)u2, (float)l);
+        };
+        if (G == 1) {
+            images([&](int n0, int n1, int n2, const double *d, double d2) {
+                if (FILL) write(total, n0, n1, n2, d, d2);
+                ++total;
+            });
+            continue;
+        }
         int cnt = 0;
         images([&](int, int, int, const double *, double) { ++cnt; });
         int incl = cnt;
         if (__ballot(cnt > 0) == 0ull) continue;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
+        for (int o = 1; o < G; o <<= 1) {
+            const int v = __shfl_up(incl, o, G);
             if (lane >= o) incl += v;
         }
         if (FILL && cnt > 0) {
             size_t at = (size_t)total + incl - cnt;
-            images([&](int n0, int n1, int n2, const double *d, double d2) {
-                // bond i -> image of j: r_ij = -d, unit vector -d / |d|
-                const double l = sqrt(d2);
-                const double u0 = -d[0] / l, u1 = -d[1] / l, u2 = -d[2] / l;
-                nbr[at] = make_int2(j, dc_pack(n0, n1, n2));
-                own[at] = i;
-                bnd64[at] = make_double4(u0, u1, u2, l);
-                bnd32[at] = make_float4((float)u0, (float)u1, (float)u2, (float)l);
-                ++at;
-            });
+            images([&](int n0, int n1, int n2, const double *d, double d2) { write(at++, n0, n1, n2, d, d2); });
         }
-        total += __shfl(incl, 63, 64);
+        total += __shfl(incl, G - 1, G);
     }
     if (!FILL && lane == 0) counts[i] = total;
-    if (__ballot(bad) != 0ull && lane == 0) atomicOr(flags, DERR_IMAGE_RANGE);
+    if (bad) atomicOr(flags, DERR_IMAGE_RANGE);
 }
 __global__ void k_bnl_tail(int n, const int *__restrict__ counts, int *__restrict__ offsets)
 {
@@ -846,8 +857,16 @@ static int batch_nl(agpu_batch *b, double rc_req)
     const int nb = (n + 255) / 256;
     AGPU_CHECK(batch_fractions(b));
     const int4 *u = b->u.as<int4>();
-    const dim3 gw((unsigned)((n + 3) / 4));
-    AGPU_LAUNCH("batch_nl_count", k_bnl<false>, gw, dim3(256), 0, s, n, b->r.as<double>(), u, G, rc,
+    // Lanes per atom by the mean size of a structure, so that small ones do not
+    // leave most lanes idle.  Both passes with 1, 8 and 64 lanes: 20 000 cells
+    // of 2 atoms 27, 57 and 217 us, of 5 67, 137 and 539 us; 4096 of 8 104, 56
+    // and 203 us; 1024 of 64 -, 76 and 115 us; 512 of 8 to 512 (mean 121) 670,
+    // 336 and 254 us.
+    const int mean = n / std::max(b->nstruct, 1), lanes = mean > 64 ? 64 : mean > 5 ? 8 : 1;
+    auto count = lanes == 64 ? k_bnl<false, 64> : lanes == 8 ? k_bnl<false, 8> : k_bnl<false, 1>;
+    auto fill = lanes == 64 ? k_bnl<true, 64> : lanes == 8 ? k_bnl<true, 8> : k_bnl<true, 1>;
+    const dim3 gw((unsigned)((n + 256 / lanes - 1) / (256 / lanes)));
+    AGPU_LAUNCH("batch_nl_count", count, gw, dim3(256), 0, s, n, b->r.as<double>(), u, G, rc,
                 nullptr, b->counts.as<int>(), nullptr, nullptr, nullptr, nullptr, flags);
     size_t tmp = 0;
     AGPU_HIP(rocprim::exclusive_scan(nullptr, tmp, b->counts.as<int>(), b->offsets.as<int>(), 0, (size_t)n,
@@ -866,7 +885,7 @@ static int batch_nl(agpu_batch *b, double rc_req)
     AGPU_CHECK(b->bnd32.reserve(sizeof(float4) * ((size_t)total + 1)));
     AGPU_CHECK(b->rev.reserve(sizeof(int) * ((size_t)total + 1)));
     AGPU_CHECK(b->own.reserve(sizeof(int) * ((size_t)total + 1)));
-    AGPU_LAUNCH("batch_nl_fill", k_bnl<true>, gw, dim3(256), 0, s, n, b->r.as<double>(), u, G, rc,
+    AGPU_LAUNCH("batch_nl_fill", fill, gw, dim3(256), 0, s, n, b->r.as<double>(), u, G, rc,
                 b->offsets.as<int>(), b->counts.as<int>(), b->nbr.as<int2>(), b->own.as<int>(), b->bnd64.as<double4>(),
                 b->bnd32.as<float4>(), flags);
     AGPU_LAUNCH("batch_nl_rev", k_bnl_rev, dim3(nb), dim3(256), 0, s, n, b->offsets.as<int>(),

@@ -216,3 +216,56 @@ def test_batch_list_edges():
         assert abs(e[s] - e0) <= 1e-10 * max(1.0, abs(e0)), s
         assert np.abs(f[a] - f0).max() <= 1e-10 * max(1.0, np.abs(f0).max()), s
     assert b.pairs() == pairs
+
+
+@pytest.mark.parametrize("sizes", [(1, 1, 2, 3, 4, 5, 9, 17), (1, 7, 8, 9, 15, 16, 17, 70, 130), (63, 64, 65, 129, 130)],
+                         ids=["one_lane", "8_lanes", "64_lanes"])
+def test_batch_list_lane_groups(sizes):
+    """The list with 1, 8 and 64 lanes per atom (chosen by the mean size up to
+    5, up to 64 and above): structures around one trip of the lanes, a number
+    of them that leaves groups of the last workgroup without an atom."""
+    from atomistica_amd.batch import TersoffBatch, params_from_theta
+    th = _theta0()
+    prm = params_from_theta(th)
+    rng = np.random.default_rng(sum(sizes))
+    S = []
+    for n in sizes:
+        edge = max(2.6, (22.0 * n) ** (1 / 3.0))
+        cell = np.diag([edge, 1.1 * edge, 0.95 * edge]) @ (np.eye(3) + rng.uniform(-0.15, 0.15, (3, 3)))
+        pos = W.random_positions(n, cell, 1.7, int(rng.integers(1 << 30)))
+        S.append((pos + rng.integers(-3, 4, (n, 3)) @ cell, cell))
+    b = TersoffBatch(S)
+    print("batch list lanes", sizes, flush=True)
+    e, f = (t.cpu().numpy() for t in b.forward(th))
+    pairs = 0
+    for s, (pos, cell) in enumerate(S):
+        # the list is built at 1.02 S
+        pairs += len(O.nl_build(pos, cell, [True] * 3, 1.02 * th[10], avgn=400)[1])
+        onl = O.nl_build(pos, cell, [True] * 3, th[10], avgn=400)
+        e0, f0 = O.tersoff(prm, pos, np.zeros(len(pos), np.int32), cell, onl)[:2]
+        a = slice(b.offsets[s], b.offsets[s + 1])
+        assert abs(e[s] - e0) <= REL * max(1.0, abs(e0)), s
+        assert np.abs(f[a] - f0).max() <= REL * max(1.0, np.abs(f0).max()), s
+    assert b.pairs() == pairs
+
+
+def test_batch_list_of_unit_cells_is_not_slow():
+    """20 000 cells of two atoms: both passes of the list take 50 us with a lane
+    per atom and took 226 us with a wavefront per atom."""
+    from atomistica_amd import native as N
+    from atomistica_amd.batch import TersoffBatch
+    rng = np.random.default_rng(3)
+    cell = np.diag([3.4, 3.4, 3.5])
+    S = [(np.array([[0, 0, 0], [1.7, 1.7, 1.75]]) + rng.normal(0, 0.05, (2, 3)), cell) for _ in range(20000)]
+    b = TersoffBatch(S)
+    best = np.inf
+    for _ in range(5):
+        N.call("agpu_batch_set_positions", b._h, N._dev(b.positions), 0)
+        N.profile_enable(True)
+        N.profile_reset()
+        b.forward(_theta0())
+        us = [1e3 * N.profile_query(k)[0] for k in ("batch_nl_count", "batch_nl_fill")]
+        N.profile_enable(False)
+        best = min(best, sum(us))
+    print("batch list of unit cells: %.1f us" % best, flush=True)
+    assert best < 110.0
