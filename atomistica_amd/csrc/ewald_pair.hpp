@@ -37,7 +37,9 @@ __device__ __forceinline__ double ewp_rcp(double x)
 // divisions, whose branches all run in a wavefront of mixed distances).
 __device__ __forceinline__ void ewp_pair(double r2, double beta, double sap, double &e, double &f)
 {
-    const double ri = rsqrt(r2), x = beta * (r2 * ri);
+    // r = 0 and no NaN at r2 = 0: coincident charges give an infinite e, as
+    // erfc(0) / 0 does
+    const double ri = rsqrt(r2), r = fmax(r2 * ri, 0.0), x = beta * r;
     const double x1 = fma(2.0, x, 1.0), xk = x + 3.75;
     const double q = ewp_rcp(x1 * xk);
     const double t = (x - 3.75) * (q * x1);
@@ -47,7 +49,7 @@ __device__ __forceinline__ void ewp_pair(double r2, double beta, double sap, dou
     const double g = exp(-(beta * beta) * r2) * ri;
     const double w = p * (q * xk);                    // exp(x^2) erfc(x)
     e = g * w;
-    f = g * (ri * ri) * fma(2.0 * sap, r2 * ri, w);   // sap = beta / sqrt(pi)
+    f = g * (ri * ri) * fma(2.0 * sap, r, w);   // sap = beta / sqrt(pi)
 }
 
 __device__ __forceinline__ void ewp_pair(double r2, float beta, float sap, double &e, double &f)

@@ -155,3 +155,29 @@ def test_real_space_ranges(n, beta, precision, rel):
         assert np.abs(fb - rf).max() <= rel * max(1.0, scale)
         assert np.abs(wb[0] - rw).max() <= rel * max(1.0, np.abs(rw).max(), np.abs(q * rp).sum())
         assert np.abs(pb - rp).max() <= rel * max(1.0, np.abs(rp).max())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_coincident_ions_give_an_infinite_energy(precision, sign):
+    """Two charges on one site: erfc(0) / 0 is infinite, so the energy is
+    infinite with the sign of the charges' product, and no NaN, in the single
+    and the batched sum and with the mesh."""
+    from atomistica_amd import native as N
+    from atomistica_amd.batch import Batch, ewald_batch
+    rng = np.random.default_rng(5)
+    cell = np.diag([14.0, 13.0, 15.0])
+    pos = rng.random((20, 3)) @ cell
+    pos[7] = pos[3]
+    q = rng.normal(size=20)
+    q[3], q[7] = 0.7, 0.7 * sign
+    q[11] -= q.sum()
+    print("coincident ions", precision, sign, flush=True)
+    for pot in (N.Ewald(cutoff=6.0, beta=0.5, kmax=2.0), N.PME(cutoff=6.0, order=6, grid=(16, 16, 16))):
+        pot.set_precision(precision)
+        p = N.from_atoms(pos, cell, [True] * 3, np.full(20, 11, np.int32))
+        nl = N.Neighbors(400)
+        pot.bind_to(p, nl)
+        assert pot.energy_and_forces(p, nl, q)[0] == sign * np.inf
+    e, f, w, phi = ewald_batch(Batch([(pos, cell)]), q, 6.0, 0.5, 2.0, precision=precision)
+    assert e.item() == sign * np.inf
