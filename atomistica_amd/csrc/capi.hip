@@ -697,6 +697,17 @@ int agpu_potential_bind_to(agpu_potential *pot, agpu_particles *p, agpu_neighbor
     return rc;
 }
 
+// Waits for a stream when a scope is left before done was set: no copy from
+// or to the caller's arrays is under way after a call that returns an error.
+struct StreamDrain {
+    hipStream_t s;
+    bool done = false;
+    ~StreamDrain()
+    {
+        if (!done) (void)hipStreamSynchronize(s);
+    }
+};
+
 static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors *nl,
                           agpu_eval_args a)
 {
@@ -770,6 +781,7 @@ static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors
     int *md = a.mask ? reinterpret_cast<int *>(cur) : nullptr;
     d.mask = md;
     hipStream_t s = stream();
+    StreamDrain drain{s};
     if (packed) {
         AGPU_CHECK(pot->h_io.wait());
         AGPU_CHECK(pot->h_io.reserve(size));
@@ -819,6 +831,7 @@ static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors
         AGPU_CHECK(pot->h_io.wait());
         AGPU_HIP(hipMemcpyAsync(h, base, sizeof(double) * back, hipMemcpyDeviceToHost, s));
         AGPU_HIP(hipStreamSynchronize(s));
+        drain.done = true;
         for (int k = 0; k < np; ++k)
             if (part[k].host) std::memcpy(part[k].host, h + (part[k].dev - base), sizeof(double) * part[k].len);
         return AGPU_OK;
@@ -827,6 +840,7 @@ static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors
         if (part[k].host && part[k].len)
             AGPU_HIP(hipMemcpyAsync(part[k].host, part[k].dev, sizeof(double) * part[k].len, hipMemcpyDeviceToHost, s));
     AGPU_HIP(hipStreamSynchronize(s));
+    drain.done = true;
     return AGPU_OK;
 }
 
