@@ -332,7 +332,7 @@ struct agpu_potential {
     void (*free_impl)(void *) = nullptr;
     agpu::DevBuf d_el, flags, partial, partial_out;
     agpu::HostStats stats;
-    // one block for the arrays of a call with host arrays
+    // blocks for the arrays of a small call with host arrays
     agpu::DevBuf io;
     agpu::HostBuf h_io;
 };

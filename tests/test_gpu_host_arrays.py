@@ -52,3 +52,26 @@ def test_no_copy_under_way_after_an_error():
     assert rc == _lib.ERR_UNSUPPORTED
     assert idle
     del b
+
+
+def test_block_of_a_large_call_is_given_back():
+    """A call with per-bond arrays needs 104 bytes per list entry on the card,
+    143 MB here, and a potential keeps the block of small calls only.  The first
+    call without them settles the memory that the potential keeps for itself."""
+    from atomistica_amd import workloads as W
+    pos, cell, pbc, Z = W.diamond_si(35, sigma=0.05, seed=2)
+    p = N.from_atoms(pos, cell, pbc, Z)
+    nl = N.Neighbors(100)
+    pot = N.Tersoff()
+    pot.bind_to(p, nl)
+    print("per-bond host arrays", len(pos), flush=True)
+    nl.update(p)
+    size = 104 * len(nl.get_list(p)[1])
+    pot.energy_and_forces(p, nl)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    pot.energy_and_forces(p, nl, epot_per_bond=True, f_per_bond=True, wpot_per_bond=True)
+    kept = before - torch.cuda.mem_get_info()[0]
+    print("  block of %.0f MB, kept %.0f MB" % (size / 1e6, kept / 1e6), flush=True)
+    assert size > 130e6
+    assert kept < 8 << 20
