@@ -42,6 +42,13 @@ namespace agpu {
 
 constexpr int PME_MAXORD = 12;
 constexpr int PME_B = 8;            // grid cells per brick edge
+// Bytes of the bricks' points that are kept at once.  A brick has p - 1 more
+// points per axis than cells, so all of them take 6.6 times the grid at order 8
+// and 13.4 times at order 12, up to 115 GB: beyond this the layers of bricks go
+// through in parts, at least one at a time (1000 x 1000 points of order 12 have
+// 0.86 GB in one).  Parts cost a little: 400^3 points of order 8, 3.4 GB, 1.95 ms
+// in one and 2.16 ms in four.
+constexpr size_t PME_BRICKS = (size_t)4 << 30;
 
 struct PmeState {
     int order = 8;
@@ -264,7 +271,7 @@ __device__ __forceinline__ void pme_brick(const PmeGrid &g, int b, int (&o)[3])
 // grid point, which looked up 64 ranges of ions for 27 ions that reach it).
 template <int ORD>
 __global__ void __launch_bounds__(64)
-k_pme_spread(PmeGrid g, CellArg B, const int *__restrict__ start, const int *__restrict__ idx,
+k_pme_spread(PmeGrid g, CellArg B, int first, const int *__restrict__ start, const int *__restrict__ idx,
              const double *__restrict__ r, const double *__restrict__ q, double *__restrict__ brick)
 {
     constexpr int E = PME_B + ORD - 1, P = pme_plane(ORD), NI = 16;
@@ -272,7 +279,7 @@ k_pme_spread(PmeGrid g, CellArg B, const int *__restrict__ start, const int *__r
     __shared__ double th[NI][3][ORD];
     __shared__ int at[NI];
     __shared__ double qs[NI];
-    const int lane = threadIdx.x, b = blockIdx.x;
+    const int lane = threadIdx.x, b = first + blockIdx.x;
     int o[3];
     pme_brick(g, b, o);
     for (int t = lane; t < E * P; t += 64) box[t] = 0.0;
@@ -315,19 +322,25 @@ k_pme_spread(PmeGrid g, CellArg B, const int *__restrict__ start, const int *__r
         }
     }
     wave_sync();
-    double *out = brick + (size_t)b * (E * E * E);
+    double *out = brick + (size_t)blockIdx.x * (E * E * E);
     for (int t = lane; t < E * E * E; t += 64) out[t] = box[t / (E * E) * P + t % (E * E)];
 }
 
 // Grid point g is in the bricks whose cells start at most p - 1 after it and
-// end no earlier than it; before the first cell the grid wraps.
-template <int ORD>
+// end no earlier than it; before the first cell the grid wraps.  PART: only the
+// bricks of layers l0 .. l1 - 1 are there, and are added to the points of the
+// nz planes that they reach.
+template <int ORD, bool PART>
 __global__ void __launch_bounds__(256)
-k_pme_merge(PmeGrid g, const double *__restrict__ brick, double *__restrict__ grid)
+k_pme_merge(PmeGrid g, int l0, int l1, int nz, const double *__restrict__ brick, double *__restrict__ grid)
 {
     constexpr int E = PME_B + ORD - 1;
-    const long long ind = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ind >= (long long)g.K[0] * g.K[1] * g.K[2]) return;
+    long long ind = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (ind >= (long long)g.K[0] * g.K[1] * nz) return;
+    if (PART) {
+        const long long plane = (long long)g.K[0] * g.K[1];
+        ind = wrapi(PME_B * l0 - (ORD - 1) + (int)(ind / plane), g.K[2]) * plane + ind % plane;
+    }
     const int p[3] = {(int)(ind % g.K[0]), (int)((ind / g.K[0]) % g.K[1]),
                       (int)(ind / ((long long)g.K[0] * g.K[1]))};
     // per axis: bricks b0 .. b1 with the point itself, then 0 .. c1 with the
@@ -343,6 +356,7 @@ k_pme_merge(PmeGrid g, const double *__restrict__ brick, double *__restrict__ gr
     double sum = 0.0;
     for (int z = 0; z < nt[2]; ++z) {
         const int bz = z < nb[2] ? b0[2] + z : z - nb[2];
+        if (PART && (bz < l0 || bz >= l1)) continue;
         const int lz = (z < nb[2] ? p[2] : p[2] - g.K[2]) - PME_B * bz + ORD - 1;
         for (int y = 0; y < nt[1]; ++y) {
             const int by = y < nb[1] ? b0[1] + y : y - nb[1];
@@ -350,12 +364,12 @@ k_pme_merge(PmeGrid g, const double *__restrict__ brick, double *__restrict__ gr
             for (int x = 0; x < nt[0]; ++x) {
                 const int bx = x < nb[0] ? b0[0] + x : x - nb[0];
                 const int lx = (x < nb[0] ? p[0] : p[0] - g.K[0]) - PME_B * bx + ORD - 1;
-                const size_t b = bx + (size_t)g.nb[0] * (by + (size_t)g.nb[1] * bz);
+                const size_t b = bx + (size_t)g.nb[0] * (by + (size_t)g.nb[1] * (PART ? bz - l0 : bz));
                 sum += brick[b * (E * E * E) + (lz * E + ly) * E + lx];
             }
         }
     }
-    grid[ind] = sum;
+    grid[ind] = PART ? grid[ind] + sum : sum;
 }
 
 // energy_and_virial_sum (pme_kernel.f90): records [e, W column-major] of
@@ -538,17 +552,30 @@ k_pme_gather(PmeGrid g, CellArg B, const int *__restrict__ start, const int *__r
     }
 }
 
+// layers of bricks whose points are kept at once
+static int pme_layers(const PmeGrid &g, int order)
+{
+    const size_t e = PME_B + order - 1, layer = sizeof(double) * e * e * e * g.nb[0] * g.nb[1];
+    return (int)std::min<size_t>(g.nb[2], std::max<size_t>(1, PME_BRICKS / layer));
+}
+
 template <int ORD>
 static int pme_spread_gather(bool gather, const PmeGrid &g, const PmeState *pm, const double *r, const double *q,
                              const CellArg &B, double fac, double *f, double *phi, hipStream_t s)
 {
-    const long long ng = (long long)g.K[0] * g.K[1] * g.K[2];
-    const unsigned nbrick = (unsigned)g.nb[0] * g.nb[1] * g.nb[2];
+    const unsigned layer = (unsigned)g.nb[0] * g.nb[1], nbrick = layer * g.nb[2];
     if (!gather) {
-        AGPU_LAUNCH("pme_spread", k_pme_spread<ORD>, dim3(nbrick), dim3(64), 0, s, g, B, pm->start.as<int>(),
-                    pm->idx_s.as<int>(), r, q, pm->brick.as<double>());
-        AGPU_LAUNCH("pme_merge", k_pme_merge<ORD>, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, s, g,
-                    pm->brick.as<double>(), pm->grid.as<double>());
+        const int nl = pme_layers(g, ORD);
+        if (nl < g.nb[2]) AGPU_CHECK(zero_dev(pm->grid.ptr, sizeof(double) * (size_t)g.K[0] * g.K[1] * g.K[2]));
+        for (int l0 = 0; l0 < g.nb[2]; l0 += nl) {
+            const int l1 = std::min(l0 + nl, g.nb[2]);
+            const int nz = nl < g.nb[2] ? std::min(PME_B * (l1 - l0) + ORD - 1, g.K[2]) : g.K[2];
+            const dim3 gm((unsigned)(((long long)g.K[0] * g.K[1] * nz + 255) / 256));
+            AGPU_LAUNCH("pme_spread", k_pme_spread<ORD>, dim3(layer * (l1 - l0)), dim3(64), 0, s, g, B, layer * l0,
+                        pm->start.as<int>(), pm->idx_s.as<int>(), r, q, pm->brick.as<double>());
+            AGPU_LAUNCH("pme_merge", (nl < g.nb[2] ? k_pme_merge<ORD, true> : k_pme_merge<ORD, false>), gm, dim3(256),
+                        0, s, g, l0, l1, nz, pm->brick.as<double>(), pm->grid.as<double>());
+        }
     } else
         AGPU_LAUNCH("pme_gather", k_pme_gather<ORD>, dim3(nbrick), dim3(256), 0, s, g, B, pm->start.as<int>(),
                     pm->idx_s.as<int>(), r, q, pm->grid.as<double>(), fac, f, phi);
@@ -630,7 +657,7 @@ int pme_recip(PmeState *pm, const agpu_particles *p, const double *q, double bet
         g.nb[d] = (pm->K[d] + PME_B - 1) / PME_B;
     }
     const int nbrick = g.nb[0] * g.nb[1] * g.nb[2];
-    const int edge = PME_B + order - 1;
+    const size_t edge = PME_B + order - 1;
     AGPU_CHECK(pm->grid.reserve(sizeof(double) * (size_t)ng));
     AGPU_CHECK(pm->spec.reserve(sizeof(double2) * (size_t)nh));
     const int nblk_g = (int)((nh + 255) / 256);
@@ -647,7 +674,7 @@ int pme_recip(PmeState *pm, const agpu_particles *p, const double *q, double bet
         AGPU_CHECK(pm->idx.reserve(sizeof(int) * (size_t)nat));
         AGPU_CHECK(pm->idx_s.reserve(sizeof(int) * (size_t)nat));
         AGPU_CHECK(pm->start.reserve(sizeof(int) * (size_t)(nbrick + 1)));
-        AGPU_CHECK(pm->brick.reserve(sizeof(double) * (size_t)nbrick * edge * edge * edge));
+        AGPU_CHECK(pm->brick.reserve(sizeof(double) * edge * edge * edge * g.nb[0] * g.nb[1] * pme_layers(g, order)));
         const dim3 ga((nat + 255) / 256);
         // The counting sort takes 4 launches (216 000 ions in 8000 bricks:
         // 25 us; the radix sort, 16 launches, 92 us).  Its scan is one

@@ -174,3 +174,42 @@ def test_pme_cluster_in_one_brick(n):
     assert ms / calls < 20.0
     again = gpu(pos, q, cell, [True] * 3, Z, 4.0, grid, 4)
     assert e == again[0] and np.array_equal(f, again[1]) and np.array_equal(phi, again[3])
+
+
+def test_pme_bricks_in_parts():
+    """Order 12 on 480 x 464 x 472 points: the bricks' points take 11 GB, of
+    which 4 GiB are kept at once, so their layers go through in three parts.  The
+    call takes those, the grid and its transform (0.8 GB each) and what the
+    transforms themselves need (bounded by 4 GB here).  More than 32 768 bricks
+    also take the radix sort.  On a mesh this fine the sum agrees with the
+    direct one."""
+    import torch
+    rng = np.random.default_rng(12)
+    cell = np.diag([30.0, 28.0, 29.0])
+    # ions next to all faces and in a layer across the middle
+    pos = np.concatenate([rng.random((100, 3)), np.round(rng.random((60, 3))) + rng.normal(0, 0.01, (60, 3)),
+                          rng.random((40, 3)) * [1, 1, 0.02] + [0, 0, 0.49]]) @ cell
+    q = rng.normal(size=200)
+    q -= q.mean()
+    cutoff = 6.0
+    beta = math.sqrt(math.log(10.0) * 12.0) / cutoff
+    print("pme bricks in parts", flush=True)
+    Z = np.full(200, 11, np.int32)
+    # the direct sum first: its memory stays with it
+    ee, fe, we, pe = gpu(pos, q, cell, [True] * 3, Z, cutoff, None, None,
+                         cls=N.Ewald(cutoff=cutoff, beta=beta, kmax=2 * beta * math.sqrt(-math.log(1e-16))))
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    p = N.from_atoms(pos, cell, [True] * 3, Z)
+    nl = N.Neighbors(400)
+    pot = N.PME(cutoff=cutoff, order=12, grid=(480, 464, 472))
+    pot.bind_to(p, nl)
+    e, f, w = pot.energy_and_forces(p, nl, q)
+    phi = pot.potential(p, nl, q)
+    grown = before - torch.cuda.mem_get_info()[0]
+    print("  memory of the call %.2f GB, dE %.1e dF %.1e" % (grown / 1e9, abs(e - ee), np.abs(f - fe).max()), flush=True)
+    assert grown < 10e9
+    assert abs(e - ee) <= REL * np.abs(q * pe).sum()
+    assert close(f, fe) and close(w, we) and close(phi, pe)
+    e2, f2, _ = pot.energy_and_forces(p, nl, q)
+    assert e2 == e and np.array_equal(f2, f)
