@@ -337,8 +337,9 @@ def _equal_oracle(pos, cell, pbc, rc, avgn):
 @pytest.mark.parametrize("n", [1, 2, 7, 63, 64, 65, 130, 700])
 @pytest.mark.parametrize("shear", [0.0, 0.25])
 def test_shared_home_atoms_of_a_bin_block(n, shear):
-    """Dense bins of few atoms in all: each block's home atoms are shared by
-    as many wavefronts as it has atoms, or as the chip still takes."""
+    """Dense bins of few atoms in all (from 63 atoms; with fewer the bins are
+    sparse and the column search takes them): each block's home atoms are shared
+    by as many wavefronts as it has atoms, or as the chip still takes."""
     rng = np.random.default_rng(n)
     cell = np.diag([11.0, 13.0, 17.5]) @ np.array([[1, 0, 0], [shear, 1, 0], [0, -shear, 1.0]])
     pos = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))) @ cell
@@ -362,3 +363,20 @@ def test_column_search(n, shear, pbc):
     if n == 300:
         q = np.concatenate([pos, (np.array([0.02, 0.5, 0.97]) + 0.02 * rng.random((120, 3))) @ cell])
         _equal_oracle(q, cell, pbc, 3.0, 400)
+
+
+@pytest.mark.parametrize("homes,shear", [(30, 0.0), (30, 0.2), (44, 0.0), (44, 0.2)])
+def test_candidates_culled_against_many_home_atoms(homes, shear):
+    """13^3 bins of 30 or 44 atoms: 30 or 22 home atoms per wavefront, whose box
+    leaves out candidates before the walk.  Random positions, some images of the
+    cell away, so the boxes are of all sizes; every row against the oracle's."""
+    rng = np.random.default_rng(homes)
+    rc, nb = 4.0, 13
+    cell = np.diag([rc * (nb + 0.1)] * 3) @ np.array([[1, 0, 0], [shear, 1, 0], [0, -shear, 1.0]])
+    # a sheared cell has bins as wide as its faces are apart
+    cell /= min(1.0, 1.0 / np.linalg.norm(np.linalg.inv(cell), axis=0).max() / (rc * (nb + 0.1)))
+    n = homes * nb ** 3
+    pos = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))) @ cell
+    print("culled candidates", homes, shear, n, flush=True)
+    _equal_oracle(pos, cell, [True] * 3, rc, 400)
+    _equal_oracle(pos - rng.integers(-1, 2, (n, 1)) * [1.0, 0.0, 0.0], cell, [False, True, True], rc, 400)

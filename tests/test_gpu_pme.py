@@ -213,3 +213,21 @@ def test_pme_bricks_in_parts():
     assert close(f, fe) and close(w, we) and close(phi, pe)
     e2, f2, _ = pot.energy_and_forces(p, nl, q)
     assert e2 == e and np.array_equal(f2, f)
+
+
+@pytest.mark.parametrize("n,grid,order", [(200, (8, 8, 8), 6), (400, (8, 16, 16), 5), (770, (16, 16, 16), 4),
+                                          (60, (136, 136, 136), 4)])
+def test_pme_sorts(n, grid, order):
+    """More than 96 ions per brick on the average take the radix sort (200 in
+    one brick, 100 in each of four; 770 in eight are just above the line); 4913
+    bricks take the one-workgroup scan a second trip."""
+    rng = np.random.default_rng(n)
+    cell = np.diag([9.0, 10.0, 12.0])
+    pos = (rng.random((n, 3)) + rng.integers(-1, 2, (n, 3))) @ cell
+    q = rng.normal(size=n)
+    q -= q.mean()
+    print("pme sorts", n, grid, order, flush=True)
+    e0, f0, w0, p0 = oracle(pos, q, cell, [True] * 3, 4.0, grid, order)
+    e, f, w, phi = gpu(pos, q, cell, [True] * 3, np.full(n, 11, np.int32), 4.0, grid, order)
+    assert abs(e - e0) <= REL * max(1.0, abs(e0))
+    assert close(f, f0) and close(w, w0) and close(phi, p0)
