@@ -91,9 +91,15 @@ struct Cell {
     int pbc[3];
 };
 
+// A number that no object and no revision had before, in any thread.  An
+// object's address may come back for another one, so what is kept from one call
+// to the next is matched by these.
+uint64_t next_rev();
+
 }  // namespace agpu
 
 struct agpu_particles {
+    const uint64_t id = agpu::next_rev();
     int nat = 0;
     int nalloc = 0;
     agpu::Cell cell{};
@@ -102,7 +108,7 @@ struct agpu_particles {
     int *d_Z = nullptr;           // (nat) device atomic numbers
     bool own_r = true, own_Z = true;
     agpu::DevBuf r_buf, Z_buf;
-    uint64_t pos_rev = 0;         // bumped on every position change
+    uint64_t pos_rev = 0;         // next_rev() on every position change
     uint64_t cell_rev = 0;
     uint64_t Z_rev = 0;
     std::vector<int> h_Z;         // host copy of atomic numbers
@@ -114,6 +120,7 @@ struct agpu_particles {
 };
 
 struct agpu_neighbors {
+    const uint64_t id = agpu::next_rev();
     int avgn = 100;
     double interaction_range = 0.0;
     double cutoff = 0.0;
@@ -124,6 +131,7 @@ struct agpu_neighbors {
     double rec[9];                // rec_cell_size, column-major image
     // provenance of the last build
     const agpu_particles *p = nullptr;
+    uint64_t p_id = 0;
     uint64_t pos_rev = ~0ull, cell_rev = ~0ull;
     int nat = 0;
     int64_t cap = 0;              // nat * avgn entries
@@ -328,6 +336,7 @@ struct agpu_potential {
     double cutoff = 0.0;          // interaction range requested at bind_to
     agpu_particles *p = nullptr;
     agpu_neighbors *nl = nullptr;
+    uint64_t p_id = 0, nl_id = 0;
     void *impl = nullptr;         // class-specific state
     void (*free_impl)(void *) = nullptr;
     agpu::DevBuf d_el, flags, partial, partial_out;
@@ -336,6 +345,21 @@ struct agpu_potential {
     agpu::DevBuf io;
     agpu::HostBuf h_io;
 };
+
+namespace agpu {
+// the list was built from, or imported for, these particles
+inline bool nl_of(const agpu_neighbors *nl, const agpu_particles *p) { return nl->p == p && nl->p_id == p->id; }
+
+inline bool bound_to(const agpu_potential *pot, const agpu_neighbors *nl)
+{
+    return pot->bound && pot->nl == nl && pot->nl_id == nl->id;
+}
+
+inline bool bound_to(const agpu_potential *pot, const agpu_particles *p, const agpu_neighbors *nl)
+{
+    return bound_to(pot, nl) && pot->p == p && pot->p_id == p->id;
+}
+}  // namespace agpu
 
 namespace agpu {
 // class hooks

@@ -187,7 +187,7 @@ extern "C" int agpu_potential_autotune(agpu_potential *pot, agpu_particles *p, a
                                        char *report, int len)
 {
     if (!pot || !p || !nl) return set_error(AGPU_ERR_ARG, "autotune: null handle");
-    if (!pot->bound || pot->p != p || pot->nl != nl)
+    if (!bound_to(pot, p, nl))
         return set_error(AGPU_ERR_STATE, "autotune: potential not bound to these objects");
     if (reps < 1) reps = 1;
     if (capturing()) return set_error(AGPU_ERR_STATE, "autotune: not during graph capture");
@@ -205,7 +205,7 @@ extern "C" int agpu_potential_set_launch(agpu_potential *pot, agpu_neighbors *nl
                                          int *nvariants)
 {
     if (!pot || !nl) return set_error(AGPU_ERR_ARG, "set_launch: null handle");
-    if (!pot->bound || pot->nl != nl)
+    if (!bound_to(pot, nl))
         return set_error(AGPU_ERR_STATE, "set_launch: potential not bound to this neighbour list");
     if (pair_mode < 0 || pair_mode > 2) return set_error(AGPU_ERR_ARG, "set_launch: pair_mode must be 0, 1 or 2");
     const bool eam = pot->kind == AGPU_KIND_EAM_ALLOY || pot->kind == AGPU_KIND_EAM;

@@ -2,9 +2,10 @@
 // per-thread error messages, the launch stream, grow-only device buffers,
 // per-kernel event timing, particles / neighbours handles and the
 // potential dispatch of init / bind_to / energy_and_forces.
+#include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
-#include <algorithm>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -43,6 +44,12 @@ hipStream_t stream()
             g_stream = nullptr;
     }
     return g_stream;
+}
+
+uint64_t next_rev()
+{
+    static std::atomic<uint64_t> rev{0};
+    return ++rev;
 }
 
 int DevBuf::reserve(size_t nbytes)
@@ -502,8 +509,8 @@ int agpu_particles_allocate(agpu_particles *p, int nat)
     AGPU_HIP(hipMemsetAsync(p->d_Z, 0, sizeof(int) * (nat + 1), stream()));
     AGPU_HIP(hipMemsetAsync(p->d_r, 0, sizeof(double) * 3 * (nat + 1), stream()));
     AGPU_HIP(hipStreamSynchronize(stream()));
-    p->pos_rev++;
-    p->Z_rev++;
+    p->pos_rev = next_rev();
+    p->Z_rev = next_rev();
     return AGPU_OK;
 }
 
@@ -514,7 +521,7 @@ int agpu_particles_set_cell(agpu_particles *p, const double *cell, const int *pb
     AGPU_CHECK(compute_inverse(cell, p->cell.B));
     for (int k = 0; k < 3; ++k) p->cell.pbc[k] = pbc ? (pbc[k] != 0) : 1;
     p->cell_set = 1;
-    p->cell_rev++;
+    p->cell_rev = next_rev();
     return AGPU_OK;
 }
 
@@ -537,7 +544,7 @@ int agpu_particles_set_atomic_numbers(agpu_particles *p, const int *Z, int flags
         AGPU_HIP(hipMemcpyAsync(p->h_Z.data(), Z, sizeof(int) * p->nat, hipMemcpyDeviceToHost, s));
     }
     AGPU_HIP(hipStreamSynchronize(s));
-    p->Z_rev++;
+    p->Z_rev = next_rev();
     return AGPU_OK;
 }
 
@@ -555,7 +562,7 @@ int agpu_particles_set_positions(agpu_particles *p, const double *r, int flags)
                                 (flags & AGPU_HOST) ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, s));
         if (flags & AGPU_HOST) AGPU_HIP(hipStreamSynchronize(s));
     }
-    p->pos_rev++;
+    p->pos_rev = next_rev();
     return AGPU_OK;
 }
 
@@ -565,14 +572,14 @@ int agpu_particles_set_position_pointer(agpu_particles *p, int nat, double *r_de
         return set_error(AGPU_ERR_ARG, "set_position_pointer: nat differs from allocate() or NULL pointer");
     p->d_r = r_device;
     p->own_r = false;
-    p->pos_rev++;
+    p->pos_rev = next_rev();
     return AGPU_OK;
 }
 
 int agpu_particles_changed_positions(agpu_particles *p)
 {
     if (!p) return set_error(AGPU_ERR_ARG, "p is NULL");
-    p->pos_rev++;
+    p->pos_rev = next_rev();
     return AGPU_OK;
 }
 
@@ -678,6 +685,8 @@ int agpu_potential_bind_to(agpu_potential *pot, agpu_particles *p, agpu_neighbor
     if (!pot || !p || !nl) return set_error(AGPU_ERR_ARG, "bind_to: NULL handle");
     pot->p = p;
     pot->nl = nl;
+    pot->p_id = p->id;
+    pot->nl_id = nl->id;
     pot->bound = 0;
     int rc = AGPU_ERR_STATE;
     switch (pot->kind) {
@@ -714,7 +723,7 @@ struct StreamDrain {
 static int stage_and_call(agpu_potential *pot, agpu_particles *p, agpu_neighbors *nl,
                           agpu_eval_args a)
 {
-    if (!pot->bound || pot->p != p || pot->nl != nl)
+    if (!bound_to(pot, p, nl))
         return set_error(AGPU_ERR_STATE, "energy_and_forces: potential not bound to these objects");
     const int nat = p->nat;
     int rc = AGPU_OK;
@@ -890,7 +899,7 @@ int agpu_coulomb_potential(agpu_potential *pot, agpu_particles *p, agpu_neighbor
     if (!pot || !p || !nl || !q || !phi) return set_error(AGPU_ERR_ARG, "potential: bad arguments");
     if (pot->kind != AGPU_KIND_EWALD && pot->kind != AGPU_KIND_PME)
         return set_error(AGPU_ERR_UNSUPPORTED, "potential: not a Coulomb class");
-    if (!pot->bound || pot->p != p || pot->nl != nl)
+    if (!bound_to(pot, p, nl))
         return set_error(AGPU_ERR_STATE, "potential: not bound to these objects");
     if (!(flags & AGPU_HOST)) return ewald_potential(pot, q, phi, 0);
     const int nat = p->nat;
@@ -949,7 +958,7 @@ static int lammps_step(agpu_potential *pot, agpu_particles *p, agpu_neighbors *n
         AGPU_CHECK(agpu_particles_set_atomic_numbers(p, Z, AGPU_HOST));
     AGPU_CHECK(agpu_particles_set_positions(p, xs.data(), AGPU_HOST));
     nl->external = false;
-    if (!pot->bound || pot->p != p || pot->nl != nl) AGPU_CHECK(agpu_potential_bind_to(pot, p, nl));
+    if (!bound_to(pot, p, nl)) AGPU_CHECK(agpu_potential_bind_to(pot, p, nl));
     if (list) AGPU_CHECK(nl_import(nl, p, seed, numneigh, neigh));
     double epot = 0.0, wpot[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     // per-atom virial: the 3x3 per atom, turned into LAMMPS' Voigt vatom with

@@ -293,7 +293,7 @@ extern "C" int agpu_md_run(agpu_md *md, int nsteps, int graph_steps, double *epo
     if (!md || nsteps < 0 || graph_steps < 0) return set_error(AGPU_ERR_ARG, "md_run: bad arguments");
     if (md->p->nat != md->nat) return set_error(AGPU_ERR_STATE, "md_run: the particles changed size");
     hipStream_t s = stream();
-    if (!md->pot->bound || md->pot->p != md->p || md->pot->nl != md->nl)
+    if (!bound_to(md->pot, md->p, md->nl))
         AGPU_CHECK(agpu_potential_bind_to(md->pot, md->p, md->nl));
     if (!md->ready) {
         // first force evaluation at the initial positions (also sizes every buffer)

@@ -1296,8 +1296,8 @@ static void geometry(const agpu_particles *p, agpu_neighbors *nl, BinGeom &g)
 bool nl_current(const agpu_neighbors *nl, const agpu_particles *p)
 {
     if (nl->pending) return false;      // a build whose flags nobody checked
-    if (nl->external || nl->held) return nl->p == p && nl->nat == p->nat;
-    return nl->p == p && nl->pos_rev == p->pos_rev && nl->cell_rev == p->cell_rev && nl->nat == p->nat;
+    if (nl->external || nl->held) return nl_of(nl, p) && nl->nat == p->nat;
+    return nl_of(nl, p) && nl->pos_rev == p->pos_rev && nl->cell_rev == p->cell_rev && nl->nat == p->nat;
 }
 
 const int *nl_flags(const agpu_neighbors *nl) { return nl->rowmax.as<int>() + 3; }
@@ -1350,17 +1350,17 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
     }
     if (nl->external) {
         // an imported list stays as the caller gave it
-        if (nl->p != p || nl->nat != p->nat)
+        if (!nl_of(nl, p) || nl->nat != p->nat)
             return set_error(AGPU_ERR_STATE, "neighbour list: imported for other particles");
         return nl_slots_refresh(nl, p);
     }
-    if (nl->held && force == 0 && nl->p == p && nl->nat == p->nat) {
+    if (nl->held && force == 0 && nl_of(nl, p) && nl->nat == p->nat) {
         AGPU_CHECK(nl_slots_refresh(nl, p));
         return csr ? nl_compact(nl) : AGPU_OK;
     }
     if (!p->cell_set) return set_error(AGPU_ERR_STATE, "particles: cell not set");
     if (p->nat > 0 && !p->d_r) return set_error(AGPU_ERR_STATE, "particles: positions not set");
-    if (!force && nl->p == p && nl->pos_rev == p->pos_rev && nl->cell_rev == p->cell_rev &&
+    if (!force && nl_of(nl, p) && nl->pos_rev == p->pos_rev && nl->cell_rev == p->cell_rev &&
         nl->nat == p->nat)
         return csr ? nl_compact(nl) : AGPU_OK;
     // invalid until this build completes
@@ -1550,6 +1550,7 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
         nl->csr = false;
         nl->caller_off = false;
         nl->p = p;
+        nl->p_id = p->id;
         nl->nat = nat;
         nl->pos_rev = p->pos_rev;
         nl->cell_rev = p->cell_rev;
@@ -1587,6 +1588,7 @@ int nl_update(agpu_neighbors *nl, agpu_particles *p, int force, bool csr, bool d
     nl->csr = nat == 0;
     nl->caller_off = nat == 0;
     nl->p = p;
+    nl->p_id = p->id;
     nl->nat = nat;
     nl->pos_rev = p->pos_rev;
     nl->cell_rev = p->cell_rev;
@@ -1679,6 +1681,7 @@ int nl_import(agpu_neighbors *nl, agpu_particles *p, const int64_t *seed, const 
     nl->external = true;
     nl->csr = true;
     nl->p = p;
+    nl->p_id = p->id;
     nl->nat = nat;
     nl->pos_rev = p->pos_rev;
     nl->cell_rev = p->cell_rev;

@@ -74,8 +74,6 @@ struct TersoffState {
     bool scr = false;
     agpu_screening_params sp;
     DevBuf keep, rcnt, roff, fcv, rkn, rco, frec, fsl, nlrev, scan_tmp;
-    int64_t nlrev_upd = -1;
-    const agpu_neighbors *nlrev_nl = nullptr;
     // take the bond-compacting path even for rows of at most 64 entries
     // (agpu_potential_set_launch variant 1 of a bond-order class)
     bool compact = false;
@@ -2086,21 +2084,14 @@ static int tersoff_scr_compute(agpu_potential *pot, const agpu_eval_args *a)
                 st->rkn.as<int>(), st->rco.as<double4>(), nullptr, dstats);
     AGPU_LAUNCH("scr_bonds", k_scr_bonds, dim3((nat + 255) / 256), dim3(256), 0, s, nat, offs, st->keep.as<int>(),
                 st->bslot.as<int>(), st->bcnt.as<int>());
-    // reverse entries of the list, once per list build
-    if (push) {
-        st->nlrev_nl = nullptr;
-    } else if (st->nlrev_nl != nl || st->nlrev_upd != nl->n_updates) {
+    // reverse entries of an imported list
+    if (!push)
         AGPU_LAUNCH("scr_rev", k_nl_rev_entries, gw, dim3(256), 0, s, nat, offs, nbr, st->nlrev.as<int>(), dstats);
-        st->nlrev_nl = nl;
-        st->nlrev_upd = nl->n_updates;
-    }
     AGPU_CHECK(int_max(st->bcnt.as<int>(), nat, dstats + 2));
     AGPU_HIP(hipMemcpyAsync(pot->stats.h, dstats, sizeof(int) * 4, hipMemcpyDeviceToHost, s));
     AGPU_HIP(hipStreamSynchronize(s));
-    if (pot->stats.h[1] & DERR_BOND_OVERFLOW) {
-        st->nlrev_nl = nullptr;
+    if (pot->stats.h[1] & DERR_BOND_OVERFLOW)
         return set_error(AGPU_ERR_NEB, "screened bond order: list entry without its reverse entry");
-    }
     const int maxb = pot->stats.h[2];
     if (maxb > 64)
         return set_error(AGPU_ERR_NEB, "screened bond order: more than 64 bonds on one atom (nebmax too small)");
@@ -2572,7 +2563,7 @@ extern "C" int agpu_potential_energy_and_forces_noalloc(agpu_potential *pot, agp
                                                         const int *mask)
 {
     if (!pot || !p || !nl || !epot || !f || !wpot) return set_error(AGPU_ERR_ARG, "noalloc: bad arguments");
-    if (!pot->bound || pot->p != p || pot->nl != nl)
+    if (!bound_to(pot, p, nl))
         return set_error(AGPU_ERR_STATE, "noalloc: potential not bound to these objects");
     switch (pot->kind) {
     case AGPU_KIND_TERSOFF:

@@ -343,3 +343,66 @@ def test_lammps_rebo2_local_energy_split():
     assert abs(eng - ep) <= REL * abs(ep)
     assert abs(ea.sum() - ep) <= REL * abs(ep)
     assert close(reverse(ea, nlocal, gown), eap) and close(reverse(f, nlocal, gown), fp)
+
+
+def test_lammps_list_screened():
+    """A screened class over LAMMPS' own list: its reverse entries are looked
+    up, not entered by the pass that finds the forces.  Three systems in a row
+    through one potential, each with handles of its own (at the addresses of
+    those before, as it happens, and with other elements), the first again at
+    the end, against the oracle's masked evaluation of the open set; and a list
+    with a one-sided entry, which is refused."""
+    from helpers import bop_cutoff
+    prm = P.Tersoff_PRB_39_5566_Si_C__Scr
+    rc = bop_cutoff(prm)
+    pot = N.TersoffScr()
+    rng = np.random.default_rng(4)
+    systems = []
+    for n, sigma in ((2, 0.2), (1, 0.1), (2, 0.3)):
+        pos, cell, _, _ = W.diamond_si(n, a=4.9, sigma=sigma, seed=n)
+        pos = _wrap(pos, cell)
+        gx, gown = ghosts(pos, cell, 4.0)
+        x = np.concatenate([pos, gx])
+        Z = np.where(rng.random(len(pos)) < 0.5, 14, 6)
+        systems.append((len(pos), x, np.concatenate([Z, Z[gown]]).astype(np.int32)))
+    for k in (0, 1, 2, 0):
+        nlocal, x, Z = systems[k]
+        print("lammps list screened", k, nlocal, len(x), flush=True)
+        lo = x.min(0)
+        box = np.diag(x.max(0) - lo + 2 * (1.0 + rc))
+        xs = x - lo + 1.0 + rc
+        el = np.array([{6: 0, 14: 1}[int(z)] for z in Z], np.int32)
+        mask = (np.arange(len(x)) < nlocal).astype(np.int32)
+        e0, f0, w0, ea0, wa0 = O.tersoff(prm, xs, el, box, O.nl_build(xs, box, [False] * 3, rc, avgn=400), mask=mask,
+                                         per_at=True)
+        lst = lammps_full_list(x, rc + 0.3)
+        e, f, v, ea = N.lammps_compute_list(pot, N.Particles(), N.Neighbors(400), nlocal, x, Z, *lst, eatom=True)
+        assert abs(e - e0) <= REL * abs(e0)
+        assert close(f, f0) and close(v, voigt(w0)) and close(ea, ea0)
+    seed, numneigh, neigh = lst
+    numneigh = numneigh.copy()
+    numneigh[3] -= 1                             # the last entry of a row
+    with pytest.raises(AgpuError):
+        N.lammps_compute_list(pot, N.Particles(), N.Neighbors(400), nlocal, x, Z, seed, numneigh, neigh)
+
+
+@pytest.mark.parametrize("own_list", [True, False])
+def test_lammps_new_handles_at_old_addresses(own_list):
+    """One potential, new particles and list handles for every step: they are
+    often at the addresses of the last ones, and nothing of those may be taken
+    for theirs (elements, the interaction range, the list)."""
+    pot = N.Tersoff()
+    case = Case("tersoff")
+    for k, (a, z) in enumerate(((4.36, 14), (3.6, 6), (5.4, 14), (4.36, 6), (3.6, 6))):
+        pos, cell, _, _ = W.diamond_si(2, a=a, sigma=0.1, seed=k)
+        Z = np.where(np.arange(len(pos)) % 3 > 0, z, 20 - z).astype(np.int32)
+        x = _wrap(pos, cell)
+        e0, f0, _, ea0, _ = case.oracle_open(x, Z, len(x))
+        print("lammps new handles", k, own_list, flush=True)
+        if own_list:
+            e, f, _, ea = N.lammps_compute(pot, N.Particles(), N.Neighbors(200), len(x), x, Z, eatom=True)
+        else:
+            e, f, _, ea = N.lammps_compute_list(pot, N.Particles(), N.Neighbors(200), len(x), x, Z,
+                                                *lammps_full_list(x, 3.5), eatom=True)
+        assert abs(e - e0) <= REL * abs(e0)
+        assert close(f, f0) and close(ea, ea0)
