@@ -250,10 +250,10 @@ struct NlShared {
 };
 
 template <bool CULL> struct NlQueue {
-    int src[NL_Q], bu[NL_Q], off[NL_Q];     // slot, bin shift and stencil offset
+    int src[NL_Q], bu[NL_Q];     // slot and bin shift
 };
 template <> struct NlQueue<false> {
-    int src[1], bu[1], off[1];
+    int src[1], bu[1];
 };
 
 // pair shift s = w_home + u_bin - w_cand; distance as the reference writes it
@@ -329,6 +329,7 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
             const int *__restrict__ cell_start, int *__restrict__ scnt,
             int2 *__restrict__ stage, int S, int *__restrict__ flags, int2 *__restrict__ part)
 {
+    static_assert(!(MULTI && CULL), "candidates of several bins' stencils are not culled");
     __shared__ NlShared sh[NL_WAVES];
     __shared__ NlQueue<CULL> shq[NL_WAVES];
     NlShared &L = sh[threadIdx.x >> 6];
@@ -507,7 +508,6 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)nq));
                         Q.src[at] = src;
                         Q.bu[at] = L.bu[b];
-                        if (MULTI) Q.off[at] = L.boff[b];
                     }
                     nq += __popcll(m);
                     // a full pass, or the last one of these bins
@@ -522,7 +522,7 @@ k_bin_pairs(int B, int nsub, BinGeom g, CellArg C, double cutoff_sq, const Sorte
                     if (CULL) {
                         src = Q.src[e];
                         bu = Q.bu[e];
-                        off = MULTI ? Q.off[e] : 0;
+                        off = 0;
                     } else {
                         const int b = find_bin(L.pre, e0 + e);
                         src = L.start[b] + e0 + e - (b ? L.pre[b - 1] : 0);
