@@ -108,6 +108,23 @@ def test_md_eam_graph_equals_stepwise(tmp_path):
     assert ca["replays"] > 0 and ca["builds"] == cb["builds"]
 
 
+def test_md_large_eam_graph_equals_stepwise(tmp_path):
+    """42 592 Cu atoms: the passes with the density table in LDS, one workgroup
+    per CU, inside a graph (from 160 atoms per CU)."""
+    fn = tmp_path / "fs_cu.eam.alloy"
+    fn.write_text(W.fs_cu_setfl_text(nr=4000, nrho=4000))
+    pos, cell, pbc, Z = W.fcc_cu(22, sigma=0.02, seed=2)
+    v = np.random.default_rng(9).normal(0.0, np.sqrt(KB * 800.0 / 63.546), pos.shape)
+    print("md large eam", len(pos), flush=True)
+    runs = []
+    for graph in (8, 0):
+        md = _md(N.TabulatedAlloyEAM(fn=str(fn)), pos, cell, pbc, Z, v, skin=0.4, masses=63.546)
+        runs.append((md.run(24, graph_steps=graph),) + md.state())
+    (ea, ra, va, fa, ca), (eb, rb, vb, fb, cb) = runs
+    assert ea == eb and np.array_equal(ra, rb) and np.array_equal(va, vb) and np.array_equal(fa, fb)
+    assert ca["replays"] > 0 and ca["builds"] == cb["builds"]
+
+
 def _bcc_w(n=3, T=900.0, seed=6):
     pos, cell = W.lattice(np.array([[0, 0, 0], [.5, .5, .5]]), n, 3.165)
     rng = np.random.default_rng(seed)
